@@ -212,6 +212,25 @@ int tccg_gett_packed_bf16(const float* A, const float* B, float* C, float alpha,
 int tccg_gett_packed_fp8(const float* A, const float* B, float* C, float alpha, float beta,
                          const tccg_gett_plan* plan, void* workspace, size_t workspace_bytes, void* stream);
 /*
+ * FP32 GETT on the BF16 MFMAs.  The packed split-BF16 kernels with FP32's
+ * contract for every input: `plan` is a split-BF16 packed plan (walk 0 or 5,
+ * no ksplit).  Where every value of a 64 x 32 pack block is 0 or has
+ * 2^-100 <= |x| < 2^51 its three BF16 parts hold it exactly; a block with any
+ * other value (infinities, NaNs, the extremes of the FP32 range) keeps its
+ * FP32 bits, and the parts of C that read it are computed on the FP32 MFMA as
+ * tccg_gett_packed_f32 computes them.  The workspace takes
+ * tccg_f32_split_workspace_bytes().  prepacked != 0: the GETT kernel alone
+ * over the operands of the previous call (A and B are not read).  The first
+ * 4 bytes at the guard region are best cleared once when the workspace is
+ * allocated (tccg_f32_split_clear_offset()): any other value there is
+ * harmless, it only makes every tile look at its guard words.
+ */
+size_t tccg_f32_split_workspace_bytes(const tccg_gett_plan* plan);
+size_t tccg_f32_split_clear_offset(const tccg_gett_plan* plan);
+int tccg_gett_f32_split(const float* A, const float* B, float* C, float alpha, float beta,
+                        const tccg_gett_plan* plan, void* workspace, size_t workspace_bytes, int prepacked,
+                        void* stream);
+/*
  * Packed GETT without allocation.  No counterpart in the reference: for
  * callers that cannot allocate device memory (code under HIP graph capture,
  * tight serving loops, harnesses that forbid hipMalloc).  Same as

@@ -15,7 +15,8 @@ from typing import Dict, Optional, Sequence, Tuple
 
 from .frontend import contraction_str, fuse_indices, parse_tccg
 from .ir import Index, Tensor
-from .plan import F32, F64, PREC_BY_NAME, PREC_NAMES, GettPlan, GettProblem, build_plan, candidate_plans, default_plan
+from .plan import (F32, F64, PREC_BY_NAME, PREC_NAMES, GettPlan, GettProblem, build_plan, call_plan,
+                   candidate_plans, default_plan, split_plans)
 
 
 def _prec_id(prec) -> int:
@@ -65,6 +66,7 @@ class Contraction:
         self.problem = GettProblem(self.C, self.A, self.B)
         self._device_plans: Dict[Tuple, object] = {}
         self._tuned: Dict[int, GettPlan] = {}
+        self._tuned_call: Dict[int, GettPlan] = {}
 
     @classmethod
     def from_tccg(cls, text: str, fuse: bool = True) -> "Contraction":
@@ -89,7 +91,9 @@ class Contraction:
 
     def plan(self, prec="f32", tile: Optional[int] = None, m_blocked: Optional[bool] = None) -> GettPlan:
         """The tuned plan (after tune()), else the model's best; an explicit
-        tile / blocking builds that plan of the gather kernel."""
+        tile / blocking builds that plan of the gather kernel.  For FP32 this
+        is a plan of the FP32 kernels (what the code generators emit); calls
+        also choose among split_plans()."""
         p = _prec_id(prec)
         if tile is None and m_blocked is None:
             return self._tuned.get(p) or default_plan(self.problem, p)
@@ -101,13 +105,23 @@ class Contraction:
     def tune(self, prec="f32", max_implementations: int = 16, inputs=None):
         """Time the best-ranked candidate plans on the GPU (tccg_amd.autotune,
         the reference's measure-and-select step, tccg/tccg.py:188-430) and make
-        the fastest this contraction's plan for `prec`; returns its measurement."""
+        the fastest this contraction's plan for `prec` (FP32: calls also choose
+        among the timed split_plans()); returns the measurement of the plan
+        that calls use."""
         from .autotune import autotune
         p = _prec_id(prec)
         best = autotune(self, p, max_implementations=max_implementations, inputs=inputs)[0]
         self._tuned[p] = best.plan
+        split = split_plans(self.problem) if p == F32 else []
+        if split:
+            best = min(best, autotune(self, p, max_implementations=max_implementations, inputs=inputs,
+                                      candidates=split)[0], key=lambda m: m.seconds)
+        self._tuned_call[p] = best.plan
         self._device_plans.pop((p, None, None), None)
         return best
+
+    def _call_plan(self, p: int) -> GettPlan:
+        return self._tuned_call.get(p) or call_plan(self.problem, p)
 
     def device_plan(self, prec="f32", tile: Optional[int] = None, m_blocked: Optional[bool] = None,
                     plan: Optional[GettPlan] = None):
@@ -118,7 +132,10 @@ class Contraction:
             key = (_prec_id(prec), tile, m_blocked)
         dp = self._device_plans.get(key)
         if dp is None:
-            dp = DevicePlan(plan if plan is not None else self.plan(prec, tile, m_blocked))
+            if plan is None:
+                plan = (self._call_plan(_prec_id(prec)) if tile is None and m_blocked is None
+                        else self.plan(prec, tile, m_blocked))
+            dp = DevicePlan(plan)
             self._device_plans[key] = dp
         return dp
 

@@ -134,6 +134,15 @@ int tccg_packed_sw_available(int prec, int tile) {
   }
 }
 
+size_t tccg_f32_split_workspace_bytes(const tccg_gett_plan* plan) {
+  return tccg_lib::f32_split_workspace_bytes(plan);
+}
+
+size_t tccg_f32_split_clear_offset(const tccg_gett_plan* plan) {
+  size_t off = 0;
+  return tccg_lib::f32_split_workspace_bytes(plan, &off) ? off : 0;
+}
+
 size_t tccg_packed_workspace_bytes(int prec, const tccg_gett_plan* plan) {
   return tccg_lib::packed_workspace_bytes(prec, plan, nullptr);
 }

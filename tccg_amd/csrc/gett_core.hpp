@@ -107,6 +107,14 @@ struct GettParams {
   // word per workgroup (1: that workgroup's partial is complete) and, after
   // them, an error word (bit 0: a wait for a partial gave up).
   uint32_t* flags;
+  // FP32 through the split-BF16 kernels (packed walks of BF16X3, gett_packed.hpp):
+  // guardAny == nullptr for plain split-BF16, else a word that is nonzero when
+  // a 64 x 32 pack block may hold its values as raw FP32 bits, and one word per
+  // pack block of A and of B (row-block major, guardK blocks along k).
+  const uint32_t* guardAny = nullptr;
+  const uint32_t* guardA = nullptr;
+  const uint32_t* guardB = nullptr;
+  int guardK = 0;
 };
 
 template <int P> struct PrecTraits;

@@ -339,6 +339,20 @@ inline size_t packed_workspace_bytes(int prec, const tccg_gett_plan* plan, size_
   return a + b + tccg::kPackedTailBytes;
 }
 
+// Workspace of FP32 through the split-BF16 kernels: that of the split-BF16
+// plan, then (256-byte aligned, before the tail that the prefetch may read) a
+// word that any raw pack block sets, padded to 256 bytes, and one guard word
+// per 64 x 32 pack block of A and of B.  0 if the plan is no packed plan.
+inline size_t f32_split_workspace_bytes(const tccg_gett_plan* plan, size_t* offG = nullptr) {
+  const size_t base = packed_workspace_bytes(tccg::BF16X3, plan, nullptr);
+  if (base == 0) return 0;
+  const size_t g = (base - tccg::kPackedTailBytes + 255) & ~(size_t)255;
+  const size_t words = ((size_t)plan->Mp / tccg::kPackTF + (size_t)plan->Np / tccg::kPackTF) *
+                       ((size_t)plan->Kp / tccg::kPackTK);
+  if (offG) *offG = g;
+  return g + 256 + ((words * 4 + 255) & ~(size_t)255) + tccg::kPackedTailBytes;
+}
+
 // Stages of the LDS ring of the packed GETT kernel.
 constexpr int kPackedStages = 3;
 
@@ -520,7 +534,8 @@ int dispatch_packed_tile(int tile, const tccg::GettParams<typename tccg::PrecTra
 template <int P, int BM, int BN, int BK>
 int run_packed_shape(const typename tccg::PrecTraits<P>::TG* A, const typename tccg::PrecTraits<P>::TG* B,
                      const tccg_gett_plan* plan, typename tccg::PrecTraits<P>::TL* wA,
-                     typename tccg::PrecTraits<P>::TL* wB, uint32_t* clear, int nclear, hipStream_t s) {
+                     typename tccg::PrecTraits<P>::TL* wB, uint32_t* clear, int nclear, uint32_t* any,
+                     hipStream_t s) {
   tccg::PackPair<typename tccg::PrecTraits<P>::TG, typename tccg::PrecTraits<P>::TL> q;
   q.X[0] = A; q.X[1] = B;
   q.offF[0] = plan->offAm; q.offF[1] = plan->offBn;
@@ -535,6 +550,11 @@ int run_packed_shape(const typename tccg::PrecTraits<P>::TG* A, const typename t
   q.kTiles = plan->Kp / BK;
   q.clear = clear;
   q.nclear = clear ? nclear : 0;
+  if (any) {   // the guard words follow it (f32_split_workspace_bytes)
+    q.any = any;
+    q.guard[0] = any + 64;
+    q.guard[1] = any + 64 + (size_t)q.nF[0] * q.nK;
+  }
   const long blocks = (long)(q.nF[0] + q.nF[1]) * q.nK;
   if (blocks > 0x7fffffff) return fail(1, "too many pack blocks");
   hipLaunchKernelGGL((tccg::pack_pair_kernel<P, BM, BN, BK>), dim3((unsigned)blocks), dim3(256), 0, s, q);
@@ -546,24 +566,26 @@ int run_packed_shape(const typename tccg::PrecTraits<P>::TG* A, const typename t
 template <int P, int I = 0>
 int pack_operands(int tile, const typename tccg::PrecTraits<P>::TG* A, const typename tccg::PrecTraits<P>::TG* B,
                   const tccg_gett_plan* plan, typename tccg::PrecTraits<P>::TL* wA,
-                  typename tccg::PrecTraits<P>::TL* wB, uint32_t* clear, int nclear, hipStream_t s) {
+                  typename tccg::PrecTraits<P>::TL* wB, uint32_t* clear, int nclear, uint32_t* any, hipStream_t s) {
   if constexpr (I >= packed_count(P)) {
     return fail(1, "invalid packed tile id");
   } else {
     constexpr TileCfg c = packed_tile(P, I);
-    if (tile == I) return run_packed_shape<P, c.BM, c.BN, c.BK>(A, B, plan, wA, wB, clear, nclear, s);
-    return pack_operands<P, I + 1>(tile, A, B, plan, wA, wB, clear, nclear, s);
+    if (tile == I) return run_packed_shape<P, c.BM, c.BN, c.BK>(A, B, plan, wA, wB, clear, nclear, any, s);
+    return pack_operands<P, I + 1>(tile, A, B, plan, wA, wB, clear, nclear, any, s);
   }
 }
 
 // pack == true: pack A and B into the workspace, then the GETT kernel;
 // pack == false: the GETT kernel alone over operands a previous call with
 // the same plan and workspace has packed (A and B are not read).
+// guard (BF16X3): FP32 results, pack blocks that the split does not hold kept
+// as raw FP32 values and their tiles computed on the FP32 MFMA.
 template <int P>
 int run_gett_packed(const typename tccg::PrecTraits<P>::TG* A, const typename tccg::PrecTraits<P>::TG* B,
                     typename tccg::PrecTraits<P>::TG* C, typename tccg::PrecTraits<P>::TG alpha,
                     typename tccg::PrecTraits<P>::TG beta, const tccg_gett_plan* plan, void* workspace,
-                    size_t workspace_bytes, void* stream, bool pack = true) {
+                    size_t workspace_bytes, void* stream, bool pack = true, bool guard = false) {
   using TG = typename tccg::PrecTraits<P>::TG;
   using TL = typename tccg::PrecTraits<P>::TL;
   if (!plan) return fail(1, "plan is NULL");
@@ -582,8 +604,9 @@ int run_gett_packed(const typename tccg::PrecTraits<P>::TG* A, const typename tc
   if (plan->Mp % tc.BM || plan->Np % tc.BN || plan->Kp % tc.BK)
     return fail(1, "table lengths must be whole multiples of the tile shape");
   if (plan->Kp % tccg::kPackTK) return fail(1, "packed plans need Kp to be a multiple of 32");
-  size_t offB = 0, offP = 0, offF = 0;
-  const size_t need = packed_workspace_bytes(P, plan, &offB, &offP, &offF);
+  size_t offB = 0, offP = 0, offF = 0, offG = 0;
+  size_t need = packed_workspace_bytes(P, plan, &offB, &offP, &offF);
+  if (guard) need = f32_split_workspace_bytes(plan, &offG);
   if (workspace_bytes < need) return fail(1, "workspace too small for the packed operands");
   // the packed kernels address elements with 32-bit offsets
   if ((offP - offB) / sizeof(TL) >= 0xffffffffull || offB / sizeof(TL) >= 0xffffffffull)
@@ -614,6 +637,17 @@ int run_gett_packed(const typename tccg::PrecTraits<P>::TG* A, const typename tc
   prm.part = reinterpret_cast<TG*>(reinterpret_cast<unsigned char*>(workspace) + offP);
   prm.flags = plan->walk == 5 ? reinterpret_cast<uint32_t*>(reinterpret_cast<unsigned char*>(workspace) + offF)
                               : nullptr;
+  uint32_t* any = nullptr;
+  if (guard) {
+    if (P != tccg::BF16X3) return fail(1, "FP32 through the split takes split-BF16 plans");
+    if ((plan->walk != 0 && plan->walk != 5) || plan->ksplit > 1)
+      return fail(1, "FP32 through the split takes packed plans of walk 0 or 5 without ksplit");
+    any = reinterpret_cast<uint32_t*>(reinterpret_cast<unsigned char*>(workspace) + offG);
+    prm.guardAny = any;
+    prm.guardK = plan->Kp / tccg::kPackTK;
+    prm.guardA = any + 64;
+    prm.guardB = any + 64 + (size_t)(plan->Mp / tccg::kPackTF) * prm.guardK;
+  }
   if (plan->ksplit < 0) return fail(1, "ksplit must be >= 0");
   if (prm.ksplit > 1) {
     if (plan->walk != 0 || (plan->grid > 0 && plan->grid < (int64_t)prm.tilesM * prm.tilesN))
@@ -647,7 +681,7 @@ int run_gett_packed(const typename tccg::PrecTraits<P>::TG* A, const typename tc
   }
   if (pack) {
     // the stream-k flags start clear: the pack launch clears them
-    int rc = pack_operands<P>(plan->tile, A, B, plan, wA, wB, prm.flags, plan->grid + 1, s);
+    int rc = pack_operands<P>(plan->tile, A, B, plan, wA, wB, prm.flags, plan->grid + 1, any, s);
     if (rc) return rc;
   }
   if (plan->walk == 4) {

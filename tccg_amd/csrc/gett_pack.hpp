@@ -95,6 +95,34 @@ template <> struct PackWriter<FP8> {
   }
 };
 
+// FP32 through the split: a value's three BF16 parts represent it exactly, and
+// the six products of two such values differ from the FP32 product by less
+// than FP32's own rounding, while every part stays a normal BF16 number and no
+// product or sum of the parts can overflow before the FP32 one does.  That
+// holds for 0 and for 2^-100 <= |x| < 2^51; infinities, NaNs and the extremes
+// of the FP32 range do not qualify.
+__device__ inline bool split_holds(float x) {
+  const uint32_t u = __float_as_uint(x);
+  return (u << 1) == 0u || ((u >> 23) & 0xffu) - 27u <= 150u;
+}
+
+// The same eight values as their FP32 bits: high halves in plane 0, low halves
+// in plane 1 (plane 2 is not read for such a block).
+__device__ inline void write8_raw(__bf16* blk, int F, int plane_stride, int r, int kin, const float* v) {
+  typedef unsigned short u16x8 __attribute__((ext_vector_type(8)));
+  u16x8 hi, lo;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const uint32_t u = __float_as_uint(v[j]);
+    hi[j] = (unsigned short)(u >> 16);
+    lo[j] = (unsigned short)u;
+  }
+  __bf16* dst = blk + chunk_pos<__bf16>(F, r, kin >> 3);
+  *reinterpret_cast<u16x8*>(dst) = hi;
+  *reinterpret_cast<u16x8*>(dst + plane_stride) = lo;
+  *reinterpret_cast<u16x8*>(dst + 2 * plane_stride) = u16x8{};
+}
+
 constexpr int kPackTF = 64;  // free positions per pack workgroup
 constexpr int kPackTK = 32;  // k positions per pack workgroup
 
@@ -106,12 +134,18 @@ constexpr int kPackTK = 32;  // k positions per pack workgroup
 // the scale maps it onto 448.
 // The 64 x 32 block at free position f0, k position k0 (tile: the
 // workgroup's LDS staging buffer).
+//
+// guard (BF16X3 only, nullptr otherwise): this block's guard word.  A block
+// with a value outside split_holds() keeps all of its values as raw FP32 bits
+// and sets its word and `any`; every other block clears its word.  `any` is
+// never cleared here: once set it only makes the GETT kernel look at the words.
 template <int P, int F, int BK>
 __device__ __forceinline__ void pack_block(const typename PrecTraits<P>::TG* __restrict__ X,
                                            const uint32_t* __restrict__ offF, const uint32_t* __restrict__ offK,
                                            int kTiles, int kfast, const float* __restrict__ amax,
                                            typename PrecTraits<P>::TL* __restrict__ out, int f0, int k0,
-                                           typename PrecTraits<P>::TG (*tile)[kPackTK + 1]) {
+                                           typename PrecTraits<P>::TG (*tile)[kPackTK + 1],
+                                           uint32_t* guard = nullptr, uint32_t* any = nullptr) {
   using TR = PrecTraits<P>;
   using TG = typename TR::TG;
   constexpr int TF = kPackTF, TK = kPackTK;
@@ -162,6 +196,22 @@ __device__ __forceinline__ void pack_block(const typename PrecTraits<P>::TG* __r
   }
   const int gf = f0 + f, gk = k0 + kl;
   const size_t blk = (size_t)(gf / F) * (size_t)kTiles * BLOCK + (size_t)(gk / BK) * BLOCK;
+  if constexpr (P == BF16X3) {
+    if (guard) {
+      bool bad = false;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) bad = bad || !split_holds(v[j]);
+      const int raw = __syncthreads_or(bad);
+      if (t == 0) {
+        *guard = raw ? 1u : 0u;
+        if (raw) *any = 1u;
+      }
+      if (raw) {
+        write8_raw(out + blk, F, F * BK, gf % F, gk % BK, v);
+        return;
+      }
+    }
+  }
   PackWriter<P>::write8(out + blk, F, F * BK, gf % F, gk % BK, v, scale);
 }
 
@@ -186,6 +236,10 @@ struct PackPair {
   int kTiles;
   uint32_t* clear;
   int nclear;
+  // FP32 through the split (BF16X3): a word per pack block of each operand
+  // (index (f0 / 64) * nK + k0 / 32) and the word that any raw block sets
+  uint32_t* guard[2] = {nullptr, nullptr};
+  uint32_t* any = nullptr;
 };
 
 template <int P, int FA, int FB, int BK>
@@ -199,10 +253,13 @@ pack_pair_kernel(PackPair<typename PrecTraits<P>::TG, typename PrecTraits<P>::TL
   const int op = lb < nA ? 0 : 1;
   if (op) lb -= nA;
   const int f0 = (lb % q.nF[op]) * kPackTF, k0 = (lb / q.nF[op]) * kPackTK;
+  uint32_t* guard = q.guard[op] ? q.guard[op] + (f0 / kPackTF) * q.nK + k0 / kPackTK : nullptr;
   if (op == 0)
-    pack_block<P, FA, BK>(q.X[0], q.offF[0], q.offK[0], q.kTiles, q.kfast[0], q.amax[0], q.out[0], f0, k0, tile);
+    pack_block<P, FA, BK>(q.X[0], q.offF[0], q.offK[0], q.kTiles, q.kfast[0], q.amax[0], q.out[0], f0, k0, tile,
+                          guard, q.any);
   else
-    pack_block<P, FB, BK>(q.X[1], q.offF[1], q.offK[1], q.kTiles, q.kfast[1], q.amax[1], q.out[1], f0, k0, tile);
+    pack_block<P, FB, BK>(q.X[1], q.offF[1], q.offK[1], q.kTiles, q.kfast[1], q.amax[1], q.out[1], f0, k0, tile,
+                          guard, q.any);
 }
 
 }  // namespace tccg

@@ -449,6 +449,99 @@ __device__ inline void sk_gather(const GettParams<typename PrecTraits<P>::TG>& p
   }
 }
 
+// FP32 through the split-BF16 kernels: whether a pack block under this wave's
+// rows of tile (tm, tn) is held as raw FP32 bits (pack_block).  guardAny is one
+// scalar load per tile; the words are read only when it is set.
+template <int BM, int BN, int WTM, int WTN>
+__device__ inline bool guard_raw(const GettParams<float>& p, int tm, int tn, int wm, int wn, int lane) {
+  if (*p.guardAny == 0u) return false;
+  const int a0 = (tm * BM + wm * WTM) >> 6, a1 = (tm * BM + wm * WTM + WTM - 1) >> 6;
+  const int b0 = (tn * BN + wn * WTN) >> 6, b1 = (tn * BN + wn * WTN + WTN - 1) >> 6;
+  uint32_t raw = 0;
+  for (int i = lane; i < (a1 - a0 + 1) * p.guardK; i += 64) raw |= p.guardA[(size_t)a0 * p.guardK + i];
+  for (int i = lane; i < (b1 - b0 + 1) * p.guardK; i += 64) raw |= p.guardB[(size_t)b0 * p.guardK + i];
+  return __any(raw != 0u);
+}
+
+// Four consecutive k values of one row of a packed block, as read from its
+// three planes; value(j) is the j-th FP32 value: the raw bits, or the sum of
+// the three parts (exact: the parts do not overlap).
+struct GuardFrag {
+  typedef unsigned short u16x4 __attribute__((ext_vector_type(4)));
+  u16x4 h, m, l;
+  bool raw;
+  template <int F, int BK>
+  __device__ inline void read(const __bf16* blk, int row, int k) {
+    const __bf16* src = blk + chunk_pos<__bf16>(F, row, k >> 3) + (k & 7);
+    h = *reinterpret_cast<const u16x4*>(src);
+    m = *reinterpret_cast<const u16x4*>(src + F * BK);
+    l = *reinterpret_cast<const u16x4*>(src + 2 * F * BK);
+  }
+  __device__ inline float value(int j) const {
+    const float x0 = __uint_as_float((uint32_t)h[j] << 16), x1 = __uint_as_float((uint32_t)m[j] << 16),
+                x2 = __uint_as_float((uint32_t)l[j] << 16);
+    return raw ? __uint_as_float(((uint32_t)h[j] << 16) | m[j]) : x0 + (x1 + x2);
+  }
+};
+
+// This wave's part of tile (tm, tn) on the FP32 MFMA, its operands rebuilt
+// from the packed planes: the result of the plain FP32 kernel (same k order,
+// same instruction) for tiles whose operands the split does not hold.  Each
+// wave reads the planes directly (no LDS, no barrier), so it can replace any
+// walk's accumulators right before their epilogue; the next eight k values are
+// in flight during the MFMAs of the current ones.
+template <int BM, int BN, int BK, int WM, int WN>
+__device__ inline void guard_recompute(const GettParams<float>& p,
+                                       Mma<BF16X3>::Acc (&acc)[TileShape<BF16X3, BM, BN, BK, WM, WN>::SN]
+                                                              [TileShape<BF16X3, BM, BN, BK, WM, WN>::SM],
+                                       int tm, int tn, int wm, int wn, int lane) {
+  using TS = TileShape<BF16X3, BM, BN, BK, WM, WN>;
+  constexpr int BLOCK_A = 3 * BM * BK, BLOCK_B = 3 * BN * BK;
+  const __bf16* Ab = reinterpret_cast<const __bf16*>(p.A) + (size_t)tm * p.kTiles * BLOCK_A;
+  const __bf16* Bb = reinterpret_cast<const __bf16*>(p.B) + (size_t)tn * p.kTiles * BLOCK_B;
+  const int K = p.kTiles * BK;
+  GuardFrag a[TS::SM], b[TS::SN];
+  auto read = [&](int k) {
+    const int kb = k / BK, kin = k - kb * BK + 4 * (lane >> 5);
+#pragma unroll
+    for (int j = 0; j < TS::SM; ++j) {
+      const int row = wm * TS::WTM + j * 32;
+      a[j].raw = p.guardA[(size_t)((tm * BM + row) >> 6) * p.guardK + (k >> 5)] != 0u;
+      a[j].template read<BM, BK>(Ab + (size_t)kb * BLOCK_A, row + (lane & 31), kin);
+    }
+#pragma unroll
+    for (int i = 0; i < TS::SN; ++i) {
+      const int row = wn * TS::WTN + i * 32;
+      b[i].raw = p.guardB[(size_t)((tn * BN + row) >> 6) * p.guardK + (k >> 5)] != 0u;
+      b[i].template read<BN, BK>(Bb + (size_t)kb * BLOCK_B, row + (lane & 31), kin);
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < TS::SN; ++i)
+#pragma unroll
+    for (int j = 0; j < TS::SM; ++j) acc[i][j] = Mma<BF16X3>::Acc{};
+  read(0);
+#pragma unroll 1
+  for (int k = 0; k < K; k += 8) {
+    float va[4][TS::SM], vb[4][TS::SN];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+#pragma unroll
+      for (int j = 0; j < TS::SM; ++j) va[s][j] = a[j].value(s);
+#pragma unroll
+      for (int i = 0; i < TS::SN; ++i) vb[s][i] = b[i].value(s);
+    }
+    read(k + 8 < K ? k + 8 : k);
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int i = 0; i < TS::SN; ++i)
+#pragma unroll
+        for (int j = 0; j < TS::SM; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(vb[s][i], va[s][j], acc[i][j], 0, 0, 0);
+  }
+}
+
 // The walk of one workgroup: tile (tm, tn), k-steps [k0, k0 + KT) (all of
 // them without a split; part ks of a split-k plan; a stream-k piece with
 // SK), and with PERSIST the tiles of work items v + gridDim.x, ... < nblocks
@@ -516,6 +609,13 @@ __device__ __forceinline__ void packed_walk(const GettParams<typename PrecTraits
   for (int i = 0; i < TS::SN; ++i)
 #pragma unroll
     for (int j = 0; j < TS::SM; ++j) acc[i][j] = typename MM::Acc{};
+  // A tile that every wave will compute on the FP32 MFMA skips the split.
+  bool all_raw = false;
+  if constexpr (P == BF16X3 && !PERSIST && !SK) {
+    if (p.guardAny && *p.guardAny != 0u)
+      all_raw = __syncthreads_and(guard_raw<BM, BN, TS::WTM, TS::WTN>(p, tm, tn, wm, wn, lane));
+    if (all_raw) KT = 0;
+  }
   // A stream-k piece that finishes its tile adds the earlier pieces' sums.
   // When its segment holds at least a tile's k-steps those were published
   // while the segment's earlier pieces ran: it starts from them, their loads
@@ -631,6 +731,10 @@ __device__ __forceinline__ void packed_walk(const GettParams<typename PrecTraits
         sk_publish<P, BM, BN, BK, WM, WN>(p, acc, sk.slot, w, lane);
         break;
       }
+    }
+    if constexpr (P == BF16X3) {
+      if (p.guardAny && guard_raw<BM, BN, TS::WTM, TS::WTN>(p, tm, tn, wm, wn, lane))
+        guard_recompute<BM, BN, BK, WM, WN>(p, acc, tm, tn, wm, wn, lane);
     }
     if (!PERSIST && ksplit > 1) {
       // raw sums of this k part into the partial-tile buffer, rows n of BM

@@ -351,6 +351,7 @@ class GettPlan:
     crun: Tuple[int, int] = (0, 0)  # packed: (E0, E1) blocks of C written as contiguous runs
     cvec: int = 0          # store-wave kernel: C written in 16-byte groups of four m positions
     ksplit: int = 1        # packed, one tile per workgroup: k range split into this many parts
+    guard: bool = False    # split-BF16 packed plan that stands in for FP32 (split_plans)
     notes: List[str] = field(default_factory=list)
 
     @property
@@ -373,9 +374,20 @@ class GettPlan:
 
     def workspace_bytes(self) -> int:
         """Device bytes of the packed operands (0 for an unpacked plan); the
-        same figure as tccg_packed_workspace_bytes()."""
+        same figure as tccg_packed_workspace_bytes(), or for a guarded plan as
+        tccg_f32_split_workspace_bytes()."""
         if not self.packed:
             return 0
+        if self.guard:
+            words = (self.Mp // 64 + self.Np // 64) * (self.Kp // PACK_TK)
+            return self._guard_offset() + 256 + -(-words * 4 // 256) * 256 + PACKED_TAIL_BYTES
+        return self._packed_bytes()
+
+    def _guard_offset(self) -> int:
+        """Where the guard words of a guarded plan's workspace begin."""
+        return -(-(self._packed_bytes() - PACKED_TAIL_BYTES) // 256) * 256
+
+    def _packed_bytes(self) -> int:
         per = _PLANES[self.prec] * _ELEM_BYTES[self.prec] * self.Kp
         ab = (-(-(per * self.Mp) // 256) * 256) + per * self.Np
         if self.walk == 5 and self.grid > 0:
@@ -406,7 +418,7 @@ class GettPlan:
         if self.ksplit > 1:
             walk += " ksplit=%d" % self.ksplit
         return ("prec=%s tile=%d (%dx%dx%d)%s%s m=%s n=%s k=%s modeA=%s modeB=%s tiles=%d Mp=%d Np=%d Kp=%d"
-                % (PREC_NAMES[self.prec], self.tile, self.BM, self.BN, self.BK, " packed" if self.packed else "",
+                % ("f32 through " + PREC_NAMES[self.prec] if self.guard else PREC_NAMES[self.prec], self.tile, self.BM, self.BN, self.BK, " packed" if self.packed else "",
                    walk, self.lin_m.inner,
                    self.lin_n.inner, self.lin_k.inner, mode[self.modeA], mode[self.modeB], self.ntiles(),
                    self.Mp, self.Np, self.Kp))
@@ -923,6 +935,15 @@ def candidate_plans(pb: GettProblem, prec: int, groupM: int = 8) -> List[GettPla
         for tile, (_, _, bk) in enumerate(VECTOR_TILES[prec]):
             if pb.K <= bk:
                 plans.append(build_vector_plan(pb, prec, tile, groupM=groupM))
+    plans += _packed_candidates(pb, prec, groupM)
+    # ties at the HBM floor are broken by the time the tile work alone would take
+    plans.sort(key=lambda p: _estimate(p))
+    return plans
+
+
+def _packed_candidates(pb: GettProblem, prec: int, groupM: int) -> List[GettPlan]:
+    """Every packed plan of candidate_plans()."""
+    plans = []
     for tile in range(len(PACKED_TILES[prec])):
         plans.append(build_packed_plan(pb, prec, tile, groupM=groupM))
         if pb.K <= 256:
@@ -950,9 +971,46 @@ def candidate_plans(pb: GettProblem, prec: int, groupM: int = 8) -> List[GettPla
             plans.append(build_packed_plan(pb, prec, tile, groupM=groupM, stream_k=1))
             if packed_ring_bytes(prec, BM, BN, BK) * 2 <= MI355X["lds_bytes_per_cu"]:
                 plans.append(build_packed_plan(pb, prec, tile, groupM=groupM, stream_k=2))
-    # ties at the HBM floor are broken by the time the tile work alone would take
+    return plans
+
+
+# Shortest k range of the plans that compute FP32 contractions on the BF16
+# MFMAs.  Their 2-norm error against FP64 is 0.45-0.88 times the FP32 MFMA's
+# for uniform, N(0, 1), positive and integer operands at every k from 4 to 5184
+# (measured; 1.25-1.4 times at k = 1, where the BF16 MFMA's truncated last
+# addition shows), and below 32 k values the packing costs more than the
+# faster instruction gains.
+SPLIT_MIN_K = 32
+
+
+def split_fits(plan: GettPlan) -> bool:
+    """The three planes of each operand stay within the 2^32 - 1 elements that
+    the packed kernels take (an FP32 operand has one plane)."""
+    return 3 * max(plan.Mp, plan.Np) * plan.Kp < 0xFFFFFF00
+
+
+def split_plans(pb: GettProblem, groupM: int = 8) -> List[GettPlan]:
+    """Guarded split-BF16 packed plans for an FP32 contraction, best model
+    estimate first: FP32 operands held exactly as three BF16 parts, the six
+    products that reach FP32's last bit, FP32 accumulation (2.4 times the FP32
+    MFMA's rate sustained), and the FP32 MFMA itself wherever an operand value
+    is not held (include/tccg_gfx950.h, tccg_gett_f32_split)."""
+    if pb.K < SPLIT_MIN_K:
+        return []
+    plans = [p for p in _packed_candidates(pb, BF16X3, groupM)
+             if p.walk in (0, 5) and p.ksplit == 1 and split_fits(p)]
+    for p in plans:
+        p.guard = True
     plans.sort(key=lambda p: _estimate(p))
     return plans
+
+
+def call_plan(pb: GettProblem, prec: int) -> GettPlan:
+    """The model's best plan to run a contraction with: default_plan(), for
+    FP32 also the plans that compute it on the BF16 MFMAs."""
+    best = default_plan(pb, prec)
+    split = split_plans(pb)[:1] if prec == F32 else []
+    return min([best] + split, key=lambda p: _estimate(p))
 
 
 def default_plan(pb: GettProblem, prec: int) -> GettPlan:

@@ -47,7 +47,8 @@ EXPORTED_SYMBOLS = ["tccg_tile_shape", "tccg_num_tiles", "tccg_gett_f32", "tccg_
                     "tccg_num_vector_tiles", "tccg_vector_tile_shape",
                     "tccg_num_transpose_tiles", "tccg_transpose_tile_shape", "tccg_transpose_f32",
                     "tccg_transpose_f64", "tccg_packed_sw_available", "tccg_gett_packed_noalloc",
-                    "tccg_gett_group"]
+                    "tccg_gett_group", "tccg_gett_f32_split", "tccg_f32_split_workspace_bytes",
+                    "tccg_f32_split_clear_offset"]
 
 _PACKED_FN = {F32: "tccg_gett_packed_f32", F64: "tccg_gett_packed_f64", BF16X3: "tccg_gett_packed_bf16x3",
               BF16: "tccg_gett_packed_bf16", FP8: "tccg_gett_packed_fp8"}
@@ -94,6 +95,12 @@ def load_library(path: Optional[Path] = None) -> ctypes.CDLL:
         lib.tccg_gett_group.restype = ctypes.c_int
         lib.tccg_packed_workspace_bytes.argtypes = [ctypes.c_int, ctypes.POINTER(_CPlan)]
         lib.tccg_packed_workspace_bytes.restype = ctypes.c_size_t
+        lib.tccg_gett_f32_split.argtypes = [vp, vp, vp, f32, f32, ctypes.POINTER(_CPlan), vp, ctypes.c_size_t,
+                                            ctypes.c_int, vp]
+        lib.tccg_gett_f32_split.restype = ctypes.c_int
+        for fn in (lib.tccg_f32_split_workspace_bytes, lib.tccg_f32_split_clear_offset):
+            fn.argtypes = [ctypes.POINTER(_CPlan)]
+            fn.restype = ctypes.c_size_t
         lib.tccg_packed_tile_shape.argtypes = lib.tccg_tile_shape.argtypes
         lib.tccg_num_packed_tiles.argtypes = [ctypes.c_int]
         lib.tccg_vector_tile_shape.argtypes = lib.tccg_tile_shape.argtypes
@@ -224,7 +231,9 @@ class DevicePlan:
         self.workspace = None
         if plan.packed:
             nbytes = plan.workspace_bytes()
-            if load_library().tccg_packed_workspace_bytes(plan.prec, ctypes.byref(c)) != nbytes:
+            lib = load_library()
+            if (lib.tccg_f32_split_workspace_bytes(ctypes.byref(c)) if plan.guard
+                    else lib.tccg_packed_workspace_bytes(plan.prec, ctypes.byref(c))) != nbytes:
                 raise GettRuntimeError("packed workspace size disagrees with the library")
             if workspace is not None:
                 if workspace.dtype != torch.uint8 or workspace.numel() < nbytes or workspace.device != dev:
@@ -233,6 +242,12 @@ class DevicePlan:
                 self.workspace = workspace
             else:
                 self.workspace = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+            if plan.guard:
+                # the word that any pack block with raw values sets: while it is
+                # clear, no tile has to look at its guard words (a copy from the
+                # host: done on return, whatever stream the first call runs on)
+                off = lib.tccg_f32_split_clear_offset(ctypes.byref(c))
+                self.workspace[off:off + 4].copy_(torch.zeros(4, dtype=torch.uint8))
 
     def _operands(self, A, B, C):
         """Tensors in the .tccg's (A, B, C) order -> kernel operands (opA, opB)."""
@@ -263,7 +278,11 @@ class DevicePlan:
                 rc = lib.tccg_amax_f32(opB.data_ptr(), opB.numel(), self.amax.data_ptr() + 4, sptr)
             if rc != 0:
                 raise GettRuntimeError(last_error())
-        if self.plan.packed:
+        if self.plan.guard:
+            rc = lib.tccg_gett_f32_split(opA.data_ptr(), opB.data_ptr(), C.data_ptr(), alpha, beta,
+                                         ctypes.byref(self.cplan), self.workspace.data_ptr(),
+                                         self.workspace.numel(), 0, sptr)
+        elif self.plan.packed:
             fn = getattr(lib, _PACKED_FN[prec])
             rc = fn(opA.data_ptr(), opB.data_ptr(), C.data_ptr(), alpha, beta, ctypes.byref(self.cplan),
                     self.workspace.data_ptr(), self.workspace.numel(), sptr)
@@ -285,9 +304,15 @@ class DevicePlan:
                      self.device)
         s = stream if stream is not None else torch.cuda.current_stream(self.device)
         with torch.cuda.device(self.device):
-            rc = load_library().tccg_gett_prepacked(self.plan.prec, C.data_ptr(), alpha, beta,
-                                                    ctypes.byref(self.cplan), self.workspace.data_ptr(),
-                                                    self.workspace.numel(), ctypes.c_void_p(s.cuda_stream))
+            lib = load_library()
+            if self.plan.guard:
+                rc = lib.tccg_gett_f32_split(None, None, C.data_ptr(), alpha, beta, ctypes.byref(self.cplan),
+                                             self.workspace.data_ptr(), self.workspace.numel(), 1,
+                                             ctypes.c_void_p(s.cuda_stream))
+            else:
+                rc = lib.tccg_gett_prepacked(self.plan.prec, C.data_ptr(), alpha, beta, ctypes.byref(self.cplan),
+                                             self.workspace.data_ptr(), self.workspace.numel(),
+                                             ctypes.c_void_p(s.cuda_stream))
         if rc != 0:
             raise GettRuntimeError("GETT launch failed: %s" % last_error())
 

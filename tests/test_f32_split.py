@@ -1,0 +1,109 @@
+"""Plans that run FP32 contractions on the BF16 MFMAs (split_plans), host side:
+which values the three parts hold, which contractions get such a plan, and the
+workspace with its guard words."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from oracle.precision_ref import split_bf16_parts
+from tccg_amd import Contraction, build
+from tccg_amd.plan import (BF16X3, F32, F64, PACKED_TAIL_BYTES, SPLIT_MIN_K, build_packed_plan, call_plan,
+                           default_plan, split_plans)
+
+
+def holds(x: np.ndarray) -> np.ndarray:
+    """split_holds() of gett_pack.hpp."""
+    u = np.ascontiguousarray(x, np.float32).view(np.uint32)
+    return ((u << np.uint32(1)) == 0) | (((u >> np.uint32(23)) & np.uint32(0xff)) - np.uint32(27) <= np.uint32(150))
+
+
+@pytest.mark.parametrize("e", [-100, -99, -1, 0, 1, 49, 50])
+def test_parts_hold_every_accepted_value(e):
+    """Every mantissa pattern class at the edges of the accepted exponents: the
+    three parts add up to the value exactly, in FP32 from the smallest up, and
+    each is zero or a normal BF16 number."""
+    rng = np.random.default_rng(e + 200)
+    man = np.concatenate([np.arange(64), (1 << 23) - 1 - np.arange(64), rng.integers(0, 1 << 23, 20000),
+                          (rng.integers(0, 128, 500) << 16) | 0x8000, (rng.integers(0, 1 << 15, 500) << 8) | 0x80])
+    x = np.concatenate([s * np.ldexp(1.0 + man / 2.0 ** 23, e) for s in (1, -1)]).astype(np.float32)
+    assert holds(x).all()
+    p0, p1, p2 = (p.astype(np.float32) for p in split_bf16_parts(x))
+    assert np.array_equal(p0 + (p1 + p2), x)
+    for p in (p0, p1, p2):
+        assert np.all((p == 0) | ((np.abs(p) >= 2.0 ** -126) & (np.abs(p) <= 2.0 ** 51)))
+
+
+def test_values_that_are_not_held():
+    x = np.array([np.inf, -np.inf, np.nan, 3e38, 2.0 ** 51, 2.0 ** -101, 1e-39, -1e-45], np.float32)
+    assert not holds(x).any()
+    assert holds(np.array([0.0, -0.0, 2.0 ** -100, np.nextafter(np.float32(2.0 ** 51), np.float32(0))], np.float32)).all()
+
+
+def _matmul(m, n, k):
+    return Contraction.from_labels(["m", "n"], ["k", "m"], ["n", "k"], {"m": m, "n": n, "k": k})
+
+
+def test_which_contractions_get_a_split_plan():
+    big = _matmul(2048, 2048, 1024)
+    assert all(p.guard and p.packed and p.prec == BF16X3 and p.walk in (0, 5) and p.ksplit == 1
+               for p in split_plans(big.problem))
+    assert call_plan(big.problem, F32).guard
+    # other precisions and the plans of the code generators are untouched
+    assert not call_plan(big.problem, BF16X3).guard and not call_plan(big.problem, F64).guard
+    assert not default_plan(big.problem, F32).guard and big.plan("f32").prec == F32
+    assert split_plans(_matmul(512, 512, SPLIT_MIN_K).problem)
+    assert not split_plans(_matmul(512, 512, SPLIT_MIN_K - 1).problem)
+
+
+@pytest.mark.parametrize("m, n, k", [(64, 64, 32), (65, 300, 33), (700, 129, 500)])
+def test_workspace_holds_the_guard_words(m, n, k):
+    path = build.library_path()
+    if not path.exists():
+        pytest.skip("library not built")
+    from tccg_amd.runtime import _CPlan, load_library
+    lib = load_library()
+    pb = _matmul(m, n, k).problem
+    for t, kw in ((0, {}), (4, {}), (5, dict(stream_k=1)), (6, dict(persistent=True))):
+        plain = build_packed_plan(pb, BF16X3, t, **kw)
+        p = build_packed_plan(pb, BF16X3, t, **kw)
+        p.guard = True
+        cp = _CPlan()
+        cp.Mp, cp.Np, cp.Kp, cp.tile, cp.walk, cp.grid = p.Mp, p.Np, p.Kp, p.tile, p.walk, p.grid
+        assert lib.tccg_f32_split_workspace_bytes(ctypes.byref(cp)) == p.workspace_bytes()
+        off = lib.tccg_f32_split_clear_offset(ctypes.byref(cp))
+        words = (p.Mp // 64 + p.Np // 64) * (p.Kp // 32)
+        # after every byte of the split-BF16 plan's, before the prefetch's tail
+        assert off % 256 == 0 and off >= plain.workspace_bytes() - PACKED_TAIL_BYTES
+        assert off + 256 + 4 * words <= p.workspace_bytes() - PACKED_TAIL_BYTES
+
+
+def test_operands_beyond_the_packed_limit_keep_the_fp32_plan():
+    """The packed planes address 2^32 - 1 elements: a contraction whose FP32
+    planes fit but whose three BF16 parts do not keeps its FP32 plan."""
+    from tccg_amd import plan as P
+    pb = _matmul(40000, 128, 40000).problem
+    assert 40000 * 40000 < 2 ** 32 - 1 < 3 * 40000 * 40000
+    assert not P.split_fits(build_packed_plan(pb, BF16X3, 0))
+    assert P.split_fits(build_packed_plan(_matmul(20000, 128, 20000).problem, BF16X3, 0))
+
+
+def test_entry_rejects_what_it_cannot_run():
+    path = build.library_path()
+    if not path.exists():
+        pytest.skip("library not built")
+    from tccg_amd.runtime import _CPlan, load_library
+    lib = load_library()
+    assert lib.tccg_gett_f32_split(None, None, None, 1.0, 0.0, None, None, 0, 0, None) != 0
+    p = build_packed_plan(_matmul(512, 512, 512).problem, BF16X3, 0)
+    cp = _CPlan()
+    cp.Mp, cp.Np, cp.Kp, cp.tile = p.Mp, p.Np, p.Kp, p.tile
+    one = ctypes.c_void_p(256)   # never dereferenced: every call below is rejected before a launch
+    for f in ("offAm", "offAk", "offBn", "offBk", "offCm", "offCn"):
+        setattr(cp, f, 256)
+    need = lib.tccg_f32_split_workspace_bytes(ctypes.byref(cp))
+    assert lib.tccg_gett_f32_split(one, one, one, 1.0, 0.0, ctypes.byref(cp), one, need - 1, 0, None) != 0
+    assert b"workspace too small" in lib.tccg_last_error()
+    cp.ksplit = 2
+    assert lib.tccg_gett_f32_split(one, one, one, 1.0, 0.0, ctypes.byref(cp), one, 1 << 40, 0, None) != 0
+    assert b"without ksplit" in lib.tccg_last_error()
