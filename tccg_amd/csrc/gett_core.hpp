@@ -526,12 +526,15 @@ __device__ inline void store_tile_from(const GettParams<typename PrecTraits<P>::
                                        typename Mma<P>::Acc (&acc)[TileShape<P, BM, BN, BK, WM, WN>::SN]
                                                                   [TileShape<P, BM, BN, BK, WM, WN>::SM],
                                        const uint32_t* cmT, const uint32_t* cnT, int wm, int wn, int lane,
-                                       float descale) {
+                                       float descale, bool checker = false) {
   using TR = PrecTraits<P>;
   using TG = typename TR::TG;
   using S = TileShape<P, BM, BN, BK, WM, WN>;
   using MM = Mma<P>;
-  const TG alpha = p.alpha, beta = p.beta;
+  // alpha by the parity of n (that of the accumulator register); checker: the
+  // accumulators hold (-1)^(m + n) C (m's parity is the lane's, pack_block)
+  const TG beta = p.beta;
+  const TG alpha[2] = {checker && (lane & 1) ? -p.alpha : p.alpha, checker && !(lane & 1) ? -p.alpha : p.alpha};
   uint32_t cm[S::SM], cn[S::SN][MM::NACC];
 #pragma unroll
   for (int j = 0; j < S::SM; ++j) {
@@ -569,8 +572,8 @@ __device__ inline void store_tile_from(const GettParams<typename PrecTraits<P>::
           TG val = (TG)acc[i][j][r];
           if (P == FP8) val = (TG)((float)val * descale);
           TG* dst = p.C + (size_t)(cm[j] + cn[i][r]);
-          if constexpr (WB) *dst = alpha * val;
-          else __builtin_nontemporal_store(alpha * val, dst);
+          if constexpr (WB) *dst = alpha[r & 1] * val;
+          else __builtin_nontemporal_store(alpha[r & 1] * val, dst);
         }
     return;
   }
@@ -586,9 +589,9 @@ __device__ inline void store_tile_from(const GettParams<typename PrecTraits<P>::
             TG val = (TG)acc[i][j][r];
             if (P == FP8) val = (TG)((float)val * descale);
             TG* dst = p.C + (size_t)(cm[j] + cn[i][r]);
-            if constexpr (!decltype(beta0)::value) *dst = alpha * val + beta * (*dst);
-            else if constexpr (WB) *dst = alpha * val;
-            else __builtin_nontemporal_store(alpha * val, dst);
+            if constexpr (!decltype(beta0)::value) *dst = alpha[r & 1] * val + beta * (*dst);
+            else if constexpr (WB) *dst = alpha[r & 1] * val;
+            else __builtin_nontemporal_store(alpha[r & 1] * val, dst);
           }
   };
   if (beta == TG(0)) update(std::true_type{});
@@ -599,8 +602,8 @@ template <int P, int BM, int BN, int BK, int WM, int WN, bool DRAIN = false>
 __device__ inline void store_tile(const GettParams<typename PrecTraits<P>::TG>& p,
                                   typename Mma<P>::Acc (&acc)[TileShape<P, BM, BN, BK, WM, WN>::SN]
                                                              [TileShape<P, BM, BN, BK, WM, WN>::SM],
-                                  int m0, int n0, int wm, int wn, int lane, float descale) {
-  store_tile_from<P, BM, BN, BK, WM, WN, DRAIN>(p, acc, p.offCm + m0, p.offCn + n0, wm, wn, lane, descale);
+                                  int m0, int n0, int wm, int wn, int lane, float descale, bool checker = false) {
+  store_tile_from<P, BM, BN, BK, WM, WN, DRAIN>(p, acc, p.offCm + m0, p.offCn + n0, wm, wn, lane, descale, checker);
 }
 
 // One BM x BN tile (tm, tn) of C over the whole k range, computed by the 256

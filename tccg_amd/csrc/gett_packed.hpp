@@ -236,7 +236,7 @@ __device__ inline void store_tile_staged(const GettParams<typename PrecTraits<P>
                                          typename Mma<P>::Acc (&acc)[TileShape<P, BM, BN, BK, WM, WN>::SN]
                                                                     [TileShape<P, BM, BN, BK, WM, WN>::SM],
                                          int m0, int n0, int wm, int wn, int lane, float descale,
-                                         unsigned char* lds_raw, int lds_bytes) {
+                                         unsigned char* lds_raw, int lds_bytes, bool checker = false) {
   using TR = PrecTraits<P>;
   using TG = typename TR::TG;
   using S = TileShape<P, BM, BN, BK, WM, WN>;
@@ -266,6 +266,7 @@ __device__ inline void store_tile_staged(const GettParams<typename PrecTraits<P>
         for (int j = 0; j < S::SM; ++j) {
           TG val = (TG)acc[i][j][r];
           if (P == FP8) val = (TG)((float)val * descale);
+          if (P == BF16X3 && checker && ((lane ^ r) & 1)) val = -val;   // store_tile_from's checker
           L[(n - p0) * LD + wm * S::WTM + j * TR::SUB + m_l] = val;
         }
       }
@@ -758,9 +759,10 @@ __device__ __forceinline__ void packed_walk(const GettParams<typename PrecTraits
       wait_vm_lgkm0<0>();  // the ring is reused for staging: every copy has landed
       __syncthreads();
       store_tile_staged<P, BM, BN, BK, WM, WN>(p, acc, tm * BM, tn * BN, wm, wn, lane, descale, smem_raw,
-                                               SH::LDS_BYTES);
+                                               SH::LDS_BYTES, P == BF16X3 && p.guardAny);
     } else {
-      store_tile<P, BM, BN, BK, WM, WN, PERSIST>(p, acc, tm * BM, tn * BN, wm, wn, lane, descale);
+      store_tile<P, BM, BN, BK, WM, WN, PERSIST>(p, acc, tm * BM, tn * BN, wm, wn, lane, descale,
+                                                 P == BF16X3 && p.guardAny);
     }
     if (!PERSIST) break;
     v += gridDim.x;

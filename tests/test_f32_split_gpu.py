@@ -124,3 +124,22 @@ def test_default_call_and_graph_replay():
         torch.cuda.synchronize()
         assert torch.equal(got.view(torch.int32), tC.view(torch.int32))
     assert torch.equal(tC, plain)
+
+
+@pytest.mark.parametrize("kw", [dict(), dict(persistent=True), dict(stream_k=1)])
+def test_sums_over_c_are_unbiased(kw):
+    """The sum of the errors over all of C, and over each of its rows and columns,
+    within five standard deviations of independent errors (their standard
+    deviation times the root of their count): a rounding to one side would leave
+    it, by the root of the count."""
+    m, n, k = 1000, 900, 240
+    c = _matmul(m, n, k)
+    A, B, C = inputs(c, 3)
+    plan = _split(c, 0, **kw)
+    out = run_gpu(c, A, B, C, prec=F32, plan=plan).astype(np.float64)
+    d = out - _exact(A, B, C, 1.0, 0.0)[0]
+    sd = d.std()
+    for axis in (None, 0, 1):
+        s = d.sum(axis=axis)
+        count = d.size if axis is None else d.shape[axis]
+        assert np.all(np.abs(s) <= 5 * sd * np.sqrt(count)), (axis, np.abs(s).max() / (sd * np.sqrt(count)))
