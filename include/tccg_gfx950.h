@@ -356,6 +356,16 @@ int tccg_gett_group(int prec, int tile, const tccg_group_operand* ops, int nops,
                     int njobs, const tccg_group_problem* problems, int nproblems, const tccg_batch_work* work,
                     int nwork, void* workspace, size_t workspace_bytes, void* stream);
 
+/* FP32 problems on the BF16 MFMAs, each with tccg_gett_f32_split's contract:
+ * the records of a TCCG_BF16X3 group, with the first 256 bytes of the
+ * workspace kept free (every `out` from 256 on; its first 4 bytes are best
+ * cleared once) and one guard word per 64 x 32 block of an operand
+ * (fBlocks * kTiles * BK / 32 words) right after the operand's planes. */
+int tccg_gett_group_f32_split(int tile, const tccg_group_operand* ops, int nops, const tccg_group_job* jobs,
+                              int njobs, const tccg_group_problem* problems, int nproblems,
+                              const tccg_batch_work* work, int nwork, void* workspace, size_t workspace_bytes,
+                              void* stream);
+
 /*
  * Tensor transposition out = alpha * permute(in) + beta * out, the step the
  * reference's TTGT method runs before and after its GEMM (Transpose,

@@ -7,10 +7,14 @@
 namespace tccg {
 
 // One 64 x 32 block per workgroup: job blockIdx.x of the list.
+//
+// guard (BF16X3: FP32 through the split, gett_pack.hpp): an operand's guard
+// words follow its planes, the word that any raw block sets begins the
+// workspace.
 template <int P, int BM, int BN, int BK>
 __global__ void __launch_bounds__(256)
 group_pack_kernel(const tccg_group_operand* __restrict__ ops, int nops, const tccg_group_job* __restrict__ jobs,
-                  int njobs, unsigned char* __restrict__ ws, size_t ws_bytes) {
+                  int njobs, unsigned char* ws, size_t ws_bytes, int guard) {
   using TR = PrecTraits<P>;
   using TG = typename TR::TG;
   using TL = typename TR::TL;
@@ -25,15 +29,19 @@ group_pack_kernel(const tccg_group_operand* __restrict__ ops, int nops, const tc
   if (Fp <= 0 || Fp % F || Kp % kPackTK || jb.f < 0 || jb.f >= op.fBlocks || jb.k < 0 || (long)jb.k * kPackTK >= Kp)
     return;
   const size_t plane = (size_t)Fp * (size_t)Kp * TR::PLANES * sizeof(TL);
-  if (op.out % 16 || op.out > ws_bytes || plane > ws_bytes - op.out) return;
+  const size_t words = guard ? (size_t)op.fBlocks * (size_t)(Kp / kPackTK) * 4 : 0;
+  if (op.out % 16 || op.out > ws_bytes || plane + words > ws_bytes - op.out || (guard && op.out < 256)) return;
+  uint32_t* word = nullptr;
+  if (guard) word = reinterpret_cast<uint32_t*>(ws + op.out + plane) + (size_t)jb.f * (Kp / kPackTK) + jb.k;
+  uint32_t* any = reinterpret_cast<uint32_t*>(ws);
   const TG* X = reinterpret_cast<const TG*>(op.X);
   TL* out = reinterpret_cast<TL*>(ws + op.out);
   if (op.isB)
     pack_block<P, BN, BK>(X, op.offF, op.offK, op.kTiles, op.kfast, nullptr, out, jb.f * kPackTF, jb.k * kPackTK,
-                          tile);
+                          tile, word, any);
   else
     pack_block<P, BM, BK>(X, op.offF, op.offK, op.kTiles, op.kfast, nullptr, out, jb.f * kPackTF, jb.k * kPackTK,
-                          tile);
+                          tile, word, any);
 }
 
 // Work item blockIdx.x: tile (tm, tn) of its problem, all k-steps, through
@@ -41,7 +49,7 @@ group_pack_kernel(const tccg_group_operand* __restrict__ ops, int nops, const tc
 template <int P, int BM, int BN, int BK, int WM, int WN, int S>
 __global__ void __launch_bounds__(256)
 gett_group_kernel(const tccg_group_problem* __restrict__ probs, int nprobs, const tccg_batch_work* __restrict__ work,
-                  int nwork, const unsigned char* __restrict__ ws, size_t ws_bytes) {
+                  int nwork, const unsigned char* __restrict__ ws, size_t ws_bytes, int guard) {
   using TR = PrecTraits<P>;
   using TG = typename TR::TG;
   using SH = PackedShape<P, BM, BN, BK, S>;
@@ -56,7 +64,10 @@ gett_group_kernel(const tccg_group_problem* __restrict__ probs, int nprobs, cons
   const size_t pa = (size_t)q.tilesM * q.kTiles * SH::BYTES_A, pb = (size_t)q.tilesN * q.kTiles * SH::BYTES_B;
   if (q.packedA % 16 || q.packedB % 16 || ws_bytes < kPackedTailBytes) return;
   const size_t lim = ws_bytes - kPackedTailBytes;
-  if (q.packedA > lim || pa > lim - q.packedA || q.packedB > lim || pb > lim - q.packedB) return;
+  const int nK = q.kTiles * BK / kPackTK;
+  const size_t ga = guard ? (size_t)q.tilesM * (BM / kPackTF) * nK * 4 : 0;
+  const size_t gb = guard ? (size_t)q.tilesN * (BN / kPackTF) * nK * 4 : 0;
+  if (q.packedA > lim || pa + ga > lim - q.packedA || q.packedB > lim || pb + gb > lim - q.packedB) return;
   GettParams<TG> p;
   p.A = reinterpret_cast<const TG*>(ws + q.packedA);
   p.B = reinterpret_cast<const TG*>(ws + q.packedB);
@@ -68,6 +79,12 @@ gett_group_kernel(const tccg_group_problem* __restrict__ probs, int nprobs, cons
   p.alpha = (TG)q.alpha; p.beta = (TG)q.beta;
   p.amax = nullptr;
   p.crunM = 0; p.crunN = 0; p.cvec = 0; p.ksplit = 1; p.part = nullptr; p.flags = nullptr;
+  if (guard) {
+    p.guardAny = reinterpret_cast<const uint32_t*>(ws);
+    p.guardA = reinterpret_cast<const uint32_t*>(ws + q.packedA + pa);
+    p.guardB = reinterpret_cast<const uint32_t*>(ws + q.packedB + pb);
+    p.guardK = nK;
+  }
   packed_walk<P, BM, BN, BK, WM, WN, S, false>(p, v, nwork, wk.tm, wk.tn, 0, 0, q.kTiles, smem_raw);
 }
 
@@ -78,19 +95,20 @@ namespace tccg_lib {
 template <int P, int I = 0>
 int launch_group(int tile, const tccg_group_operand* ops, int nops, const tccg_group_job* jobs, int njobs,
                  const tccg_group_problem* probs, int nprobs, const tccg_batch_work* work, int nwork, void* ws,
-                 size_t ws_bytes, hipStream_t s) {
+                 size_t ws_bytes, int guard, hipStream_t s) {
   if constexpr (I >= packed_count(P)) {
     return fail(1, "invalid packed tile id");
   } else {
     constexpr TileCfg c = packed_tile(P, I);
     if (tile != I)
-      return launch_group<P, I + 1>(tile, ops, nops, jobs, njobs, probs, nprobs, work, nwork, ws, ws_bytes, s);
+      return launch_group<P, I + 1>(tile, ops, nops, jobs, njobs, probs, nprobs, work, nwork, ws, ws_bytes, guard,
+                                    s);
     constexpr int ST = kPackedStages;
     using SH = tccg::PackedShape<P, c.BM, c.BN, c.BK, ST>;
     unsigned char* wsb = reinterpret_cast<unsigned char*>(ws);
     if (njobs > 0) {
       hipLaunchKernelGGL((tccg::group_pack_kernel<P, c.BM, c.BN, c.BK>), dim3(njobs), dim3(256), 0, s, ops, nops,
-                         jobs, njobs, wsb, ws_bytes);
+                         jobs, njobs, wsb, ws_bytes, guard);
       hipError_t e = hipGetLastError();
       if (e != hipSuccess) return fail((int)e, std::string("group pack launch: ") + hipGetErrorString(e));
     }
@@ -99,7 +117,7 @@ int launch_group(int tile, const tccg_group_operand* ops, int nops, const tccg_g
       static std::atomic<uint64_t> lds_set{0};
       if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kern), SH::LDS_BYTES, lds_set)) return rc;
       hipLaunchKernelGGL(kern, dim3(nwork), dim3(256), SH::LDS_BYTES, s, probs, nprobs, work, nwork,
-                         (const unsigned char*)wsb, ws_bytes);
+                         (const unsigned char*)wsb, ws_bytes, guard);
       hipError_t e = hipGetLastError();
       if (e != hipSuccess) return fail((int)e, std::string("group GETT launch: ") + hipGetErrorString(e));
     }
@@ -110,7 +128,7 @@ int launch_group(int tile, const tccg_group_operand* ops, int nops, const tccg_g
 template <int P>
 int run_group(int tile, const tccg_group_operand* ops, int nops, const tccg_group_job* jobs, int njobs,
               const tccg_group_problem* probs, int nprobs, const tccg_batch_work* work, int nwork, void* ws,
-              size_t ws_bytes, void* stream) {
+              size_t ws_bytes, void* stream, int guard = 0) {
   if (nops < 0 || njobs < 0 || nprobs < 0 || nwork < 0) return fail(1, "negative count");
   if ((njobs > 0 && (!ops || !jobs || nops == 0)) || (nwork > 0 && (!probs || !work || nprobs == 0)))
     return fail(1, "group array is NULL or empty");
@@ -120,7 +138,7 @@ int run_group(int tile, const tccg_group_operand* ops, int nops, const tccg_grou
   packed_tiles_of(P, &ntiles);
   if (tile < 0 || tile >= ntiles) return fail(1, "invalid packed tile id");
   return launch_group<P>(tile, ops, nops, jobs, njobs, probs, nprobs, work, nwork, ws, ws_bytes,
-                         (hipStream_t)stream);
+                         guard, (hipStream_t)stream);
 }
 
 }  // namespace tccg_lib

@@ -65,7 +65,12 @@ class GettGroup:
     workspace) and launch() as often as needed; the tensors' pointers are
     baked in."""
 
-    def __init__(self, prec: int, tile: int, order: str = "xcd"):
+    def __init__(self, prec: int, tile: int, order: str = "xcd", guard: bool = False):
+        """guard: FP32 problems on the split-BF16 kernels (prec BF16X3) with
+        FP32's contract for every value (tccg_gett_group_f32_split)."""
+        if guard and prec != BF16X3:
+            raise ValueError("FP32 through the split runs on the split-BF16 kernels")
+        self.guard = guard
         if order not in ("xcd", "lpt"):
             raise ValueError("work order is 'xcd' or 'lpt'")
         self.order = order
@@ -124,11 +129,17 @@ class GettGroup:
                             locality if locality is not None else (a, b)))
         return len(self._probs) - 1
 
+    def _header(self) -> int:
+        """Bytes before the first operand: the word that any raw block sets."""
+        return 256 if self.guard else 0
+
     def plane_bytes(self, op) -> int:
-        return op[5] * op[6] * _PLANES[self.prec] * _ELEM_BYTES[self.prec]
+        n = op[5] * op[6] * _PLANES[self.prec] * _ELEM_BYTES[self.prec]
+        # a guard word per pack block after the planes
+        return n + 4 * (op[5] // PACK_TF) * (op[6] // PACK_TK) if self.guard else n
 
     def workspace_bytes(self) -> int:
-        total = 0
+        total = self._header()
         for op in self._ops:
             total += -(-self.plane_bytes(op) // 256) * 256
         return total + PACKED_TAIL_BYTES
@@ -204,7 +215,7 @@ class GettGroup:
         tables = np.concatenate(chunks) if chunks else np.zeros(4, np.int32)
         tptr = [table_base + 4 * o for o in offs]
         ops = (_COperand * max(1, len(self._ops)))()
-        out_off, jobs, pos = [], [], 0
+        out_off, jobs, pos = [], [], self._header()
         for i, (ptr, tF, tK, kf, isb, Fp, Kp) in enumerate(self._ops):
             o = ops[i]
             o.X, o.offF, o.offK, o.out = ptr, tptr[tF], tptr[tK], pos
@@ -237,6 +248,8 @@ class GettGroup:
             workspace = torch.empty(need, dtype=torch.uint8, device=dev)
         elif workspace.dtype != torch.uint8 or workspace.numel() < need or workspace.device != dev:
             raise ValueError("group workspace must be a uint8 tensor of >= %d bytes on %s" % (need, dev))
+        if self.guard:
+            workspace[:4].copy_(torch.zeros(4, dtype=torch.uint8))
         up = lambda arr: torch.from_numpy(np.frombuffer(bytes(arr), dtype=np.uint8).copy()).to(dev)
         self._bound = dict(tables=tables, ops=up(ops), nops=len(self._ops), jobs=torch.from_numpy(jobs).to(dev),
                            njobs=int(jobs.shape[0]), probs=up(probs), nprobs=len(self._probs),
@@ -254,10 +267,11 @@ class GettGroup:
         s = stream if stream is not None else torch.cuda.current_stream(dev)
         vp = ctypes.c_void_p
         with torch.cuda.device(dev):
-            rc = b["lib"].tccg_gett_group(self.prec, self.tile, vp(b["ops"].data_ptr()), b["nops"],
-                                          vp(b["jobs"].data_ptr()), b["njobs"], vp(b["probs"].data_ptr()),
-                                          b["nprobs"], vp(b["work"].data_ptr()), b["nwork"],
-                                          vp(b["ws"].data_ptr()), b["ws"].numel(), vp(s.cuda_stream))
+            args = (self.tile, vp(b["ops"].data_ptr()), b["nops"], vp(b["jobs"].data_ptr()), b["njobs"],
+                    vp(b["probs"].data_ptr()), b["nprobs"], vp(b["work"].data_ptr()), b["nwork"],
+                    vp(b["ws"].data_ptr()), b["ws"].numel(), vp(s.cuda_stream))
+            rc = (b["lib"].tccg_gett_group_f32_split(*args) if self.guard
+                  else b["lib"].tccg_gett_group(self.prec, *args))
         if rc != 0:
             raise GettRuntimeError("grouped GETT failed: %s" % b["lib"].tccg_last_error().decode())
 
@@ -270,9 +284,10 @@ def group_for_plans(plans: Sequence, As, Bs, Cs, alphas: Sequence[float], betas:
     if not plans:
         raise ValueError("empty group")
     prec, tile = plans[0].prec, plans[0].tile
-    g = GettGroup(prec, tile, order)
+    guard = plans[0].guard
+    g = GettGroup(prec, tile, order, guard)
     for p, A, B, C, al, be in zip(plans, As, Bs, Cs, alphas, betas):
-        if p.prec != prec or p.tile != tile or not p.packed or p.ksplit > 1 or p.walk != 0:
+        if p.prec != prec or p.tile != tile or p.guard != guard or not p.packed or p.ksplit > 1 or p.walk != 0:
             raise ValueError("group plans must be one-tile packed plans of one precision and tile")
         opA, opB = (B, A) if p.problem.swapped else (A, B)
         a = g.operand(opA.data_ptr(), p.offAm, p.offAk, kfast(p.modeA), False)

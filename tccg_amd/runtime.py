@@ -47,7 +47,7 @@ EXPORTED_SYMBOLS = ["tccg_tile_shape", "tccg_num_tiles", "tccg_gett_f32", "tccg_
                     "tccg_num_vector_tiles", "tccg_vector_tile_shape",
                     "tccg_num_transpose_tiles", "tccg_transpose_tile_shape", "tccg_transpose_f32",
                     "tccg_transpose_f64", "tccg_packed_sw_available", "tccg_gett_packed_noalloc",
-                    "tccg_gett_group", "tccg_gett_f32_split", "tccg_f32_split_workspace_bytes",
+                    "tccg_gett_group", "tccg_gett_f32_split", "tccg_gett_group_f32_split", "tccg_f32_split_workspace_bytes",
                     "tccg_f32_split_clear_offset"]
 
 _PACKED_FN = {F32: "tccg_gett_packed_f32", F64: "tccg_gett_packed_f64", BF16X3: "tccg_gett_packed_bf16x3",
@@ -93,6 +93,8 @@ def load_library(path: Optional[Path] = None) -> ctypes.CDLL:
         lib.tccg_gett_group.argtypes = [ctypes.c_int, ctypes.c_int, vp, ctypes.c_int, vp, ctypes.c_int, vp,
                                         ctypes.c_int, vp, ctypes.c_int, vp, ctypes.c_size_t, vp]
         lib.tccg_gett_group.restype = ctypes.c_int
+        lib.tccg_gett_group_f32_split.argtypes = lib.tccg_gett_group.argtypes[1:]
+        lib.tccg_gett_group_f32_split.restype = ctypes.c_int
         lib.tccg_packed_workspace_bytes.argtypes = [ctypes.c_int, ctypes.POINTER(_CPlan)]
         lib.tccg_packed_workspace_bytes.restype = ctypes.c_size_t
         lib.tccg_gett_f32_split.argtypes = [vp, vp, vp, f32, f32, ctypes.POINTER(_CPlan), vp, ctypes.c_size_t,

@@ -126,6 +126,34 @@ def test_default_call_and_graph_replay():
     assert torch.equal(tC, plain)
 
 
+@pytest.mark.parametrize("order", ["xcd", "lpt"])
+@pytest.mark.parametrize("shape", [(128, 128, 16), (192, 192, 16), (192, 64, 16)])
+def test_grouped_problems_with_special_values(shape, order):
+    """A group of uneven problems, raw blocks in some operands: every problem
+    against FP64 with the bound of the single call, special values as plain FP32."""
+    import torch
+    from tccg_amd.batch import GettBatch
+    sizes = [(333, 290, 104), (64, 64, 4), (200, 131, 37), (333, 290, 104)]
+    cs = [_matmul(*s) for s in sizes]
+    ops = [inputs(c, 20 + i, with_c=True) for i, c in enumerate(cs)]
+    ops[3] = _specials(*ops[3][:2]) + (ops[3][2],)
+    alphas, betas = [1.0, 1.5, -0.5, 1.5], [0.0, 0.5, 0.0, 0.5]
+    dev = lambda x: torch.from_numpy(np.ascontiguousarray(x)).cuda()
+    As, Bs, Cs = ([dev(o[i]) for o in ops] for i in range(3))
+    b = GettBatch(cs, alphas=alphas, betas=betas, group_tile=PACKED_TILES[F32].index(shape), group_order=order)
+    assert all(p.guard for p in b.plans)
+    b.bind(As, Bs, Cs).launch()
+    torch.cuda.synchronize()
+    for (m, n, k), (A, B, C), got, al, be in zip(sizes, ops, Cs, alphas, betas):
+        out = got.cpu().numpy()
+        ref, mag = _exact(A, B, C, al, be)
+        fp32 = run_gpu(_matmul(m, n, k), A, B, C, prec=F32, alpha=al, beta=be,
+                       plan=build_packed_plan(_matmul(m, n, k).problem, F32, 2))
+        assert np.array_equal(np.isnan(out), np.isnan(fp32)) and np.array_equal(np.isinf(out), np.isinf(fp32))
+        ok = np.isfinite(out)
+        assert np.all(np.abs(out[ok] - ref[ok]) <= (k + 8) * 2.0 ** -23 * mag[ok] + 2.0 ** -125)
+
+
 @pytest.mark.parametrize("kw", [dict(), dict(persistent=True), dict(stream_k=1)])
 def test_sums_over_c_are_unbiased(kw):
     """The sum of the errors over all of C, and over each of its rows and columns,
