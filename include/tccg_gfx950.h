@@ -409,6 +409,12 @@ int tccg_transpose_f64(const double* in, double* out, double alpha, double beta,
 /* out[0] = max_i |x[i]| (device float); used for the FP8 per-tensor scales. */
 int tccg_amax_f32(const float* x, int64_t n, float* out, void* stream);
 
+/* out[0] = max|A|, out[1] = max|B| in one launch.  out: a device array of
+ * tccg_amax_pair_floats() floats, zero before its first use and then left to
+ * these calls, which run one after the other. */
+size_t tccg_amax_pair_floats(void);
+int tccg_amax_pair_f32(const float* A, int64_t nA, const float* B, int64_t nB, float* out, void* stream);
+
 /* Message of the last failed call on this thread ("" if none). */
 const char* tccg_last_error(void);
 

@@ -33,6 +33,70 @@ __global__ void amax_kernel(const float* __restrict__ x, int64_t n, unsigned* ou
   }
 }
 
+// Blocks per operand of amax_pair_kernel at most: enough loads in flight for
+// the whole chip (1024 threads per CU), few enough that the last block reduces
+// their maxima in one load per thread.
+constexpr int kAmaxBlocks = 512;
+
+__device__ inline float block_max(float m, float* red) {
+  for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_down(m, off, 64));
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+  __syncthreads();
+  m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+  __syncthreads();
+  return m;
+}
+
+// max|A| and max|B| in one launch: blocks [0, nbA) walk A, the rest B; each
+// stores its maximum, and the block that finishes last reduces them all, so
+// nothing has to be cleared beforehand.  What bounds it is latency, not bytes:
+// as two clears and two reductions (one atomic per block on the result word)
+// it took four launches and 26 us before the FP8 pack launch of 2 x 5.3 MB;
+// one launch takes 6 us.  Scratch: out[0..1], the count of finished blocks
+// (wraps to 0 by itself), then kAmaxBlocks maxima per operand.
+__global__ void __launch_bounds__(256)
+amax_pair_kernel(const float* __restrict__ A, int64_t nA, const float* __restrict__ B, int64_t nB, int nbA,
+                 float* out) {
+  __shared__ float red[4];
+  __shared__ int last;
+  unsigned* done = reinterpret_cast<unsigned*>(out + 2);
+  float* part = out + 4;
+  const bool second = (int)blockIdx.x >= nbA;
+  const float* x = second ? B : A;
+  const int64_t n = second ? nB : nA;
+  const int b = second ? blockIdx.x - nbA : blockIdx.x;
+  const int64_t stride = (int64_t)(second ? gridDim.x - nbA : nbA) * 256;
+  const int64_t first = (int64_t)b * 256 + threadIdx.x;
+  float m = 0.f;
+  // 16-byte loads from the first aligned element on; |x| compares as before
+  const int64_t head = (4 - ((reinterpret_cast<uintptr_t>(x) >> 2) & 3)) & 3;
+  const int64_t quads = n > head ? (n - head) / 4 : 0;
+  const float4* q = reinterpret_cast<const float4*>(x + head);
+  for (int64_t i = first; i < quads; i += stride) {
+    const float4 v = q[i];
+    m = fmaxf(fmaxf(m, fmaxf(fabsf(v.x), fabsf(v.y))), fmaxf(fabsf(v.z), fabsf(v.w)));
+  }
+  const int64_t rest = n - quads * 4;   // at most 6 elements, before and after the quads
+  if (first < rest) m = fmaxf(m, fabsf(first < head ? x[first] : x[quads * 4 + first]));
+  m = block_max(m, red);
+  if (threadIdx.x == 0) {
+    __hip_atomic_store(part + (second ? kAmaxBlocks : 0) + b, m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __threadfence();
+    last = atomicInc(done, gridDim.x - 1) == gridDim.x - 1;
+  }
+  __syncthreads();
+  if (!last) return;
+  __threadfence();
+  for (int op = 0; op < 2; ++op) {
+    const int nb = op ? gridDim.x - nbA : nbA;
+    float v = 0.f;
+    for (int i = threadIdx.x; i < nb; i += 256)
+      v = fmaxf(v, __hip_atomic_load(part + op * kAmaxBlocks + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    v = block_max(v, red);
+    if (threadIdx.x == 0) out[op] = v;
+  }
+}
+
 }  // namespace
 
 }  // namespace tccg_lib
@@ -181,6 +245,20 @@ int tccg_amax_f32(const float* x, int64_t n, float* out, void* stream) {
   int64_t blocks = (n + 255) / 256;
   if (blocks > 256) blocks = 256;
   hipLaunchKernelGGL(amax_kernel, dim3((unsigned)blocks), dim3(256), 0, s, x, n, reinterpret_cast<unsigned*>(out));
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return fail((int)e, std::string("amax launch: ") + hipGetErrorString(e));
+  return 0;
+}
+
+size_t tccg_amax_pair_floats(void) { return 4 + 2 * (size_t)tccg_lib::kAmaxBlocks; }
+
+int tccg_amax_pair_f32(const float* A, int64_t nA, const float* B, int64_t nB, float* out, void* stream) {
+  using namespace tccg_lib;
+  if (!A || !B || !out || nA <= 0 || nB <= 0) return fail(1, "amax: bad arguments");
+  // 4096 elements (four 16-byte loads per thread) per block
+  auto blocks = [](int64_t n) { return (int)std::min<int64_t>((n + 4095) / 4096, kAmaxBlocks); };
+  const int nbA = blocks(nA), nbB = blocks(nB);
+  hipLaunchKernelGGL(amax_pair_kernel, dim3(nbA + nbB), dim3(256), 0, (hipStream_t)stream, A, nA, B, nB, nbA, out);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail((int)e, std::string("amax launch: ") + hipGetErrorString(e));
   return 0;

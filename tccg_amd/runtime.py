@@ -48,7 +48,7 @@ EXPORTED_SYMBOLS = ["tccg_tile_shape", "tccg_num_tiles", "tccg_gett_f32", "tccg_
                     "tccg_num_transpose_tiles", "tccg_transpose_tile_shape", "tccg_transpose_f32",
                     "tccg_transpose_f64", "tccg_packed_sw_available", "tccg_gett_packed_noalloc",
                     "tccg_gett_group", "tccg_gett_f32_split", "tccg_gett_group_f32_split", "tccg_f32_split_workspace_bytes",
-                    "tccg_f32_split_clear_offset"]
+                    "tccg_f32_split_clear_offset", "tccg_amax_pair_f32", "tccg_amax_pair_floats"]
 
 _PACKED_FN = {F32: "tccg_gett_packed_f32", F64: "tccg_gett_packed_f64", BF16X3: "tccg_gett_packed_bf16x3",
               BF16: "tccg_gett_packed_bf16", FP8: "tccg_gett_packed_fp8"}
@@ -108,6 +108,8 @@ def load_library(path: Optional[Path] = None) -> ctypes.CDLL:
         lib.tccg_vector_tile_shape.argtypes = lib.tccg_tile_shape.argtypes
         lib.tccg_num_vector_tiles.argtypes = [ctypes.c_int]
         lib.tccg_amax_f32.argtypes = [vp, ctypes.c_int64, vp, vp]
+        lib.tccg_amax_pair_f32.argtypes = [vp, ctypes.c_int64, vp, ctypes.c_int64, vp, vp]
+        lib.tccg_amax_pair_floats.restype = ctypes.c_size_t
         from .transpose import TRANSPOSE_TILES, _CTransposePlan
         for name, T in (("tccg_transpose_f32", f32), ("tccg_transpose_f64", f64)):
             fn = getattr(lib, name)
@@ -211,7 +213,10 @@ class DevicePlan:
         i32 = np.int32
         self.tables = [up(plan.offAm, i32), up(plan.offAk, i32), up(plan.offBn, i32), up(plan.offBk, i32),
                        up(plan.offCm, i32), up(plan.offCn, i32), up(plan.ordA, i32), up(plan.ordB, i32)]
-        self.amax = torch.zeros(2, dtype=torch.float32, device=dev) if plan.prec == FP8 else None
+        # max|A|, max|B| and the reduction's scratch (cleared from the host: done
+        # on return, whatever stream the first call runs on)
+        self.amax = (torch.zeros(load_library().tccg_amax_pair_floats(), dtype=torch.float32).to(dev)
+                     if plan.prec == FP8 else None)
         c = _CPlan()
         (c.offAm, c.offAk, c.offBn, c.offBk, c.offCm, c.offCn, c.ordA, c.ordB) = [t.data_ptr() for t in self.tables]
         c.Mp, c.Np, c.Kp = plan.Mp, plan.Np, plan.Kp
@@ -275,9 +280,8 @@ class DevicePlan:
         sptr = ctypes.c_void_p(s.cuda_stream)
         prec = self.plan.prec
         if prec == FP8:
-            rc = lib.tccg_amax_f32(opA.data_ptr(), opA.numel(), self.amax.data_ptr(), sptr)
-            if rc == 0:
-                rc = lib.tccg_amax_f32(opB.data_ptr(), opB.numel(), self.amax.data_ptr() + 4, sptr)
+            rc = lib.tccg_amax_pair_f32(opA.data_ptr(), opA.numel(), opB.data_ptr(), opB.numel(),
+                                        self.amax.data_ptr(), sptr)
             if rc != 0:
                 raise GettRuntimeError(last_error())
         if self.plan.guard:
