@@ -238,6 +238,16 @@ class Linearization:
     def offsets(self, tensor: Tensor, pad_to: int = 1) -> np.ndarray:
         """uint32 element offsets of `tensor` along this linearisation; INVALID
         where a position holds no element."""
+        if self.is_plain():
+            # column-major order of the whole set: outer sums, no coordinates
+            off = np.zeros(1, dtype=np.int64)
+            for l, e in zip(self.labels, self.extents):
+                off = (np.arange(e, dtype=np.int64)[:, None] * max(0, tensor.stride_of_label(l)) + off).reshape(-1)
+            if off.size and off.max(initial=0) >= 0xFFFFFFFF:
+                raise UnsupportedContraction("tensor %s exceeds 2^32-1 elements" % tensor.label)
+            out = np.full(-(-off.size // pad_to) * pad_to, INVALID, dtype=np.uint32)
+            out[:off.size] = off
+            return out
         coord, valid = self.coords(pad_to)
         off = np.zeros(coord.shape[0], dtype=np.int64)
         for i, l in enumerate(self.labels):
@@ -477,9 +487,7 @@ def _store_run(offCm: np.ndarray, offCn: np.ndarray, BM: int) -> int:
     cm = offCm.astype(np.int64)
     if cm.size == 0 or cm[0] == np.int64(INVALID):
         return 0
-    R = 1
-    while R < cm.size and cm[R] == cm[0] + R:
-        R += 1
+    R = _leading_run(cm, 1)
     if R % 4 or R >= BM or BM % R or cm.size % R:
         return 0
     t = cm.reshape(-1, R)
@@ -780,19 +788,49 @@ def store_efficiency(segment_bytes: float) -> float:
     return 0.75 * min(1.0, max(segment_bytes, 16.0) / 1024.0) ** 0.3
 
 
+# Constants of the launch estimate, fitted (least squares on the logarithm,
+# plans near their contraction's best weighted up) to 17091 timed plans of 114
+# contractions: every pattern of tccg_amd.workloads over extents 8-72 (96-384
+# for the short-k pattern), every candidate plan.  The model's first choice
+# takes 1.04 (FP32), 1.02 (split-BF16), 1.04 (BF16), 1.04 (FP64) and 1.02 (FP8)
+# times the best candidate's time in the geometric mean, where the constants
+# before took 1.59, 1.42, 1.27, 1.15 and 1.06; the worst choice 1.95 times (5.2
+# before: store waves over a handful of tiles).
+#
+# Packed kernels, per precision: MFMA time of a k-step over the nominal peak
+# (`mfma`), the share of the k-step's LDS traffic (128 bytes per clock) that the
+# MFMAs do not hide (`lds`), the shortest k-step of a workgroup in us (`step`),
+# a tile's prologue and epilogue in us (`tile`), the time of storing a tile over
+# what its CU's share of HBM bandwidth gives (`store`), and how much slower the
+# MFMAs run with every CU busy, where the power limit lowers the clock (`power`).
+_PACKED_COST = {
+    F32: dict(mfma=1.08, lds=0.15, step=0.42, tile=2.0, store=0.18, power=0.04),
+    F64: dict(mfma=1.13, lds=0.3, step=0.23, tile=1.3, store=0.18, power=0.05),
+    BF16X3: dict(mfma=1.0, lds=0.29, step=0.36, tile=2.2, store=0.235, power=0.37),
+    FP8: dict(mfma=1.58, lds=0.0, step=0.07, tile=8.5, store=0.32, power=0.03),
+    BF16: dict(mfma=1.0, lds=0.35, step=0.21, tile=1.2, store=0.23, power=0.76),
+}
+# Gather kernels: the same, `scalar` the slowdown per operand read in a scalar
+# load mode, `walk` the us a persistent workgroup spends between tiles.
+_GATHER_COST = {
+    F32: dict(mfma=1.71, step=1.11, tile=0.75, store=0.29, scalar=0.13, walk=0.0),
+    F64: dict(mfma=1.94, step=0.90, tile=0.59, store=0.22, scalar=0.0, walk=1.29),
+    BF16X3: dict(mfma=3.33, step=1.33, tile=0.48, store=0.33, scalar=0.19, walk=0.12),
+    FP8: dict(mfma=8.3, step=0.88, tile=0.0, store=0.73, scalar=3.0, walk=0.0),
+    BF16: dict(mfma=8.6, step=0.80, tile=0.56, store=0.335, scalar=0.41, walk=0.0),
+}
+_CALL_US, _LAUNCH_US = 10.9, 2.9    # a call back to back with others: its first launch, every other one
+_PACK_US, _PACK_BW = 6.2, 4.5e12    # the pack launch with the gap after it; bytes/s it moves
+
+
 def _c_segment_bytes(plan: GettPlan) -> float:
     """Contiguous bytes of C a store instruction of the plan's epilogue writes."""
     esz = 8 if plan.prec == F64 else 4
     cm = plan.offCm.astype(np.int64)
-    L = 1
-    while L < min(cm.size, 4096) and cm[L] == cm[0] + L:
-        L += 1
+    L = _leading_run(cm[:4096], 1)
     if plan.walk == 4:
         if plan.crun[0]:
-            cn = plan.offCn.astype(np.int64)[:plan.BN]
-            adj = 1
-            while adj < cn.size and cn[adj] == cn[adj - 1] + plan.crun[0]:
-                adj += 1
+            adj = _leading_run(plan.offCn.astype(np.int64)[:plan.BN], plan.crun[0])
             return min(1024.0, plan.crun[0] * adj * esz)
         return min(L, plan.BM) * esz if plan.cvec else esz
     if plan.packed and plan.crun[0] and (not plan.grid or plan.walk == 5):
@@ -801,116 +839,170 @@ def _c_segment_bytes(plan: GettPlan) -> float:
     return min(L, sub) * esz
 
 
-def _tile_costs(plan: GettPlan, beta: float = 0.0):
-    """Per-tile pieces of the launch estimate: (workgroup slots on the GPU,
-    MFMA time of one tile on one slot, its fixed cost, the pack kernels'
-    time, its C write-back time)."""
-    hw = MI355X
+def _line_stores(plan: GettPlan) -> float:
+    """Share of C's row segments (the 32 or 16 consecutive m positions of one
+    MFMA column block) that are whole, aligned 128-byte lines."""
     esz = 8 if plan.prec == F64 else 4
-    if plan.walk == 4:
-        lds = sw_lds_bytes(plan.prec, plan.BM, plan.BN, plan.BK)
-    else:
-        lds = (packed_ring_bytes(plan.prec, plan.BM, plan.BN, plan.BK) if plan.packed
-               else lds_bytes(plan.prec, plan.BM, plan.BN, plan.BK))
-    per_cu = max(1, min(2, hw["lds_bytes_per_cu"] // lds))
-    slots = hw["cus"] * per_cu
-    eff = 0.75 if plan.BM * plan.BN >= 128 * 128 else 0.55
-    t_pack = 0.0
-    if plan.packed:
-        # contiguous tile copies, no per-tile conversion; the pack kernels read
-        # each operand once and write its planes once
-        eff = 0.88 if plan.BM * plan.BN >= 192 * 192 else 0.85 if plan.BM * plan.BN >= 128 * 128 else 0.6
-        if plan.walk == 4:
-            eff *= 0.92   # the staged tile's LDS writes and the store waves' issue slots
-        src = 8 if plan.prec == F64 else 4
-        moved = (src + _PLANES[plan.prec] * _ELEM_BYTES[plan.prec]) * (plan.Mp + plan.Np) * plan.Kp
-        t_pack = 6.0e-6 + moved / (0.6 * hw["hbm_bytes_per_s"])
-    else:
-        if plan.modeA in (FREE1, KDIM1):
-            eff *= 0.85
-        if plan.modeB in (FREE1, KDIM1):
-            eff *= 0.85
-        # operands split or quantised again for every tile that reads them
-        eff *= {BF16X3: 0.45, BF16: 0.6, FP8: 0.6}.get(plan.prec, 1.0)
-    t_mfma = 2.0 * plan.BM * plan.BN * plan.Kp / plan.ksplit / (hw["peak"][plan.prec] / slots) / eff
-    if plan.packed:
-        # LDS traffic per tile: every k-step's copy into the ring plus the four
-        # waves' fragment reads (each wave reads its half of A's and B's rows),
-        # and for the store-wave kernel the staged tile written and read once;
-        # 128 bytes per clock per CU
-        ring = 3.0 * _PLANES[plan.prec] * _ELEM_BYTES[plan.prec] * (plan.BM + plan.BN) * plan.Kp / plan.ksplit
-        staged = 2.0 * 4 * plan.BM * plan.BN if plan.walk == 4 else 0.0
-        t_lds = (ring + staged) / (128 * hw["clock_ghz"] * 1e9) * (hw["cus"] / slots)
-        # measured: the compute waves' LDS traffic adds to their MFMA time when
-        # it is comparable (short k-steps of small wave tiles)
-        t_mfma = max(t_mfma, t_lds) + (min(t_mfma, t_lds) if plan.walk == 4 else 0.0)
-    seff = store_efficiency(_c_segment_bytes(plan))
-    t_store = esz * plan.BM * plan.BN / (seff * hw["hbm_bytes_per_s"] / slots)
-    t_fixed = 2.0e-6 + t_store
-    if plan.walk == 2:
-        t_fixed = 0.1e-6 + t_store * 0.5
-    elif plan.grid:
-        t_fixed = 0.4e-6 + t_store * 0.6
-    return slots, t_mfma, t_fixed, t_pack, t_store
+    sub = 16 if plan.prec in (FP8, F64) else 32
+    if sub * esz < 128:
+        return 0.0
+    cm = plan.offCm.astype(np.int64)
+    seg = cm[:cm.size // sub * sub].reshape(-1, sub)
+    held = (seg != np.int64(INVALID)).any(axis=1)
+    whole = held & (seg - seg[:, :1] == np.arange(sub)).all(axis=1)
+    cn = plan.offCn.astype(np.int64)
+    cn = cn[cn != np.int64(INVALID)]
+    start = seg[whole, 0]
+    if not start.size or not cn.size:
+        return 0.0
+    pick = lambda a: a[np.linspace(0, a.size - 1, 499).astype(np.int64)] if a.size > 499 else a
+    aligned = np.mean((pick(start)[:, None] + pick(cn)[None, :]) % (128 // esz) == 0)
+    return float(np.count_nonzero(whole) / np.count_nonzero(held) * aligned)
+
+
+def _occupancy(plan: GettPlan) -> int:
+    """Workgroups of the plan's kernel resident on one CU (LDS, then registers)."""
+    area = plan.BM * plan.BN
+    if not plan.packed:
+        return 1 if area >= 128 * 128 else 2
+    ring = packed_ring_bytes(plan.prec, plan.BM, plan.BN, plan.BK)
+    by_regs = 1 if area >= 192 * 192 else 2 if area >= 128 * 128 else 4
+    return max(1, min(by_regs, MI355X["lds_bytes_per_cu"] // ring))
+
+
+def _pack_us(plan: GettPlan) -> float:
+    """The pack launch: each operand read once, its planes written once."""
+    if not plan.packed:
+        return 0.0
+    src = 8 if plan.prec == F64 else 4
+    moved = (src + _PLANES[plan.prec] * _ELEM_BYTES[plan.prec]) * (plan.Mp + plan.Np) * plan.Kp
+    return _PACK_US + moved / _PACK_BW * 1e6
+
+
+def _tile_store_us(plan: GettPlan, beta: float) -> float:
+    """HBM time of a tile of C at one CU's share of the bandwidth."""
+    esz = 8 if plan.prec == F64 else 4
+    share = MI355X["hbm_bytes_per_s"] / MI355X["cus"]
+    return esz * plan.BM * plan.BN / (share * store_efficiency(_c_segment_bytes(plan))) * (2 if beta != 0 else 1) * 1e6
+
+
+def _step_us(plan: GettPlan, busy: float) -> float:
+    """One k-step of one workgroup with the CU's matrix cores to itself; busy:
+    share of the GPU's CUs that hold a workgroup."""
+    peak = MI355X["peak"][plan.prec] / MI355X["cus"]
+    mfma = 2.0 * plan.BM * plan.BN * plan.BK / peak * 1e6
+    if not plan.packed:
+        c = _GATHER_COST[plan.prec]
+        scalar = (plan.modeA in (FREE1, KDIM1)) + (plan.modeB in (FREE1, KDIM1))
+        return mfma * c["mfma"] * (1.0 + c["scalar"] * scalar)
+    c = _PACKED_COST[plan.prec]
+    # the ring's copies and the four waves' fragment reads
+    lds = 3.0 * _PLANES[plan.prec] * _ELEM_BYTES[plan.prec] * (plan.BM + plan.BN) * plan.BK
+    return (mfma * c["mfma"] * (1.0 + c["power"] * busy)
+            + c["lds"] * lds / (128 * MI355X["clock_ghz"] * 1e3))
+
+
+def _rounds_us(items: int, slots: int, steps: float, step: float, shortest: float, tile: float,
+               store: float) -> float:
+    """items tiles of `steps` k-steps over the CUs, `slots` resident on each:
+    the busiest CU runs whole rounds of `slots` and a last one of the rest.
+    Resident workgroups share the matrix cores and the CU's bandwidth."""
+    def tiles(j):
+        return steps * max(shortest, j * step) + tile + j * store if j else 0.0
+    rounds, rest = divmod(-(-items // MI355X["cus"]), slots)
+    return rounds * tiles(slots) + tiles(rest)
 
 
 def group_estimate(plans: Sequence[GettPlan], betas: Optional[Sequence[float]] = None) -> float:
     """Estimate of one grouped launch over packed one-tile plans: every tile
-    of every plan shares the GPU's workgroup slots (no per-problem rounds),
-    plus one pack launch moving every operand once."""
+    of every plan shares the GPU (no per-problem rounds), plus one pack
+    launch moving every operand once."""
     betas = list(betas) if betas is not None else [0.0] * len(plans)
     t, t_pack = 0.0, 0.0
     for p, b in zip(plans, betas):
-        slots, t_mfma, t_fixed, tp, _ = _tile_costs(p, b)
-        t += p.ntiles() * (t_mfma + t_fixed) / slots
-        t_pack += max(0.0, tp - 6.0e-6)
-    return t + t_pack + 6.0e-6
+        c, slots = _PACKED_COST[p.prec], _occupancy(p)
+        per = (p.Kp // p.BK * max(c["step"], slots * _step_us(p, 1.0)) + c["tile"]
+               + slots * c["store"] * _tile_store_us(p, b))
+        t += p.ntiles() * per / (slots * MI355X["cus"])
+        t_pack += _pack_us(p) - _PACK_US
+    return (t + t_pack + _PACK_US) * 1e-6
 
 
 def _estimate(plan: GettPlan, beta: float = 0.0) -> Tuple[float, float]:
-    """Estimate of one launch, the gfx950 analogue of Gett.estimateGFLOPS
-    (tccg/gett.py:590-687): per tile, MFMA time of the padded work plus a fixed
-    cost (gather latency and C write-back at the slot's share of HBM
-    bandwidth; mostly hidden by the persistent walk), times the number of
-    tile rounds over the CUs; bounded below by the HBM time of A, B and C."""
-    pb = plan.problem
-    hw = MI355X
+    """Estimate of one call, the gfx950 analogue of Gett.estimateGFLOPS
+    (tccg/gett.py:590-687), in seconds: (the time a caller sees, the GPU's):
+    launches of small contractions are paced by the host, and plans equal in
+    that are ordered by the GPU's time."""
+    pb, hw = plan.problem, MI355X
+    cus = hw["cus"]
     esz = 8 if plan.prec == F64 else 4
-    if plan.walk == 3:
-        # HBM time of A, B and C against the FMAs on the vector ALUs (one FMA
-        # per lane per cycle, half issued).  With four-wide groups C is written
-        # in whole-kilobyte runs, the best store pattern there is: no tile work
-        # beyond the HBM floor, so it wins ties there.  Scalar groups store one
-        # element per lane per instruction.
-        bytes_ = esz * (pb.opA.size() + pb.opB.size() + pb.C.size() * (2 if beta != 0 else 1))
-        eff = 0.8 if plan.modeA == FREE4 else 0.45
-        t_hbm = bytes_ / (eff * hw["hbm_bytes_per_s"])
-        t_valu = plan.padded_flops() / (0.5 * hw["valu"][plan.prec])
-        t = max(t_hbm, t_valu)
-        return t, (0.0 if plan.modeA == FREE4 else t)
-    slots, t_mfma, t_fixed, t_pack, t_store = _tile_costs(plan, beta)
-    ntiles = plan.ntiles() * plan.ksplit
-    rounds = ntiles / slots if plan.grid else math.ceil(ntiles / slots)
-    if plan.walk == 5:
-        # the tile work spread evenly over the machine; each workgroup walks
-        # about one piece more than its share of tiles (a pipeline start and
-        # an epilogue each) and publishes and adds one partial tile, mostly
-        # behind other workgroups' MFMAs
-        t_part = 2.0 * esz * plan.BM * plan.BN / (0.6 * hw["hbm_bytes_per_s"] / plan.grid)
-        t = (ntiles * t_mfma / slots + (ntiles / plan.grid + 1.0) * t_fixed * min(1.0, slots / plan.grid)
-             + 0.25 * t_part + t_pack)
-    elif plan.walk == 4:
-        # store waves write C while the compute waves run the next tile: the
-        # slower of the two per tile, plus staging the tile through LDS
-        t = rounds * (max(t_mfma, t_store) + 0.3e-6) + t_pack
-    else:
-        t = rounds * (t_mfma + t_fixed) + t_pack
-    if plan.ksplit > 1:
-        # the reduction reads ksplit partial tiles and writes C once
-        t += 3e-6 + (plan.ksplit + 1) * esz * plan.Mp * plan.Np / (0.6 * hw["hbm_bytes_per_s"])
     bytes_ = esz * (pb.opA.size() + pb.opB.size() + pb.C.size() * (2 if beta != 0 else 1))
-    t_hbm = bytes_ / (0.8 * hw["hbm_bytes_per_s"])
-    return max(t, t_hbm), t
+    if plan.walk == 3:
+        # HBM time of A, B and C, written in whole-kilobyte runs with four-wide
+        # groups and element by element without, against the FMAs on the vector
+        # ALUs (one FMA per lane per cycle, half issued)
+        eff = ((0.67, 0.5) if plan.prec == F64 else (0.84, 0.58))[plan.modeA != FREE4]
+        gpu = 1.5 + 1e6 * max(bytes_ / (eff * hw["hbm_bytes_per_s"]),
+                              plan.padded_flops() / (0.5 * hw["valu"][plan.prec]))
+        return max(gpu, _CALL_US) * 1e-6, gpu * 1e-6
+    n = plan.ntiles() * plan.ksplit
+    steps = plan.Kp / plan.BK / plan.ksplit
+    slots = _occupancy(plan)
+    # with the CUs idle for part of the last round the clock stays higher
+    step = _step_us(plan, n / (cus * -(-n // cus)))
+    store = _tile_store_us(plan, beta)
+    launches = 1
+    if not plan.packed:
+        c = _GATHER_COST[plan.prec]
+        if plan.walk == 2 or plan.grid:
+            grid = max(1, min(plan.grid, cus * slots))
+            j = max(1.0, grid / cus)
+            gpu = (-(-n // grid) * (steps * max(c["step"], j * step) + c["walk"] + 1.8 * j * c["store"] * store)
+                   + c["tile"])
+        else:
+            # non-temporal stores of partial lines go to HBM part by part
+            gpu = _rounds_us(n, slots, steps, step, c["step"], c["tile"],
+                             c["store"] * store * (1.0 + 1.2 * (1.0 - _line_stores(plan))))
+    else:
+        c = _PACKED_COST[plan.prec]
+        launches = 3 if plan.ksplit > 1 else 2
+        tile_store = c["store"] * store
+        partial = tile_store
+        if plan.walk in (0, 5) and (not plan.grid or plan.walk == 5):
+            if plan.crun[0]:   # the run epilogue's passes through LDS
+                partial = tile_store + 1.3 * store
+            else:              # non-temporal stores, as above
+                partial = tile_store * (1.0 + 1.25 * (1.0 - _line_stores(plan)))
+        if plan.walk == 5:
+            # the k-steps spread evenly over the grid; each workgroup walks
+            # about a piece more than its share of tiles, and publishes and
+            # adds one partial tile
+            per_cu = max(1.0, plan.grid / cus)
+            # (pieces of distant tiles share fewer blocks in L2: more power)
+            step = _step_us(plan, 1.2)
+            gpu = (n * steps / plan.grid * max(c["step"], min(per_cu, slots) * step) * max(1.0, per_cu / slots)
+                   + 5.2 + c["tile"] + (n / plan.grid + 1.0) * partial
+                   + 2.5 * esz * plan.BM * plan.BN * plan.grid / 4.8e6)
+        elif plan.walk == 4:
+            # store waves write C while the compute waves run the next tile;
+            # part of the shorter of the two still adds to the longer
+            out = tile_store * (1.3 if _c_segment_bytes(plan) < 16 else 1.0)
+            gpu = (math.ceil(max(1.0, n / plan.grid))
+                   * (max(1.16 * steps * max(c["step"], step), 1.5 * out) + 2.0 * min(steps * step, out) + 0.87)
+                   + c["tile"] + out)
+        elif plan.grid:
+            grid = max(1, min(plan.grid, cus * slots))
+            j = max(1.0, grid / cus)
+            gpu = -(-n // grid) * (steps * max(c["step"], j * step) + 0.5 + 1.8 * j * tile_store) + c["tile"]
+        else:
+            gpu = _rounds_us(n, slots, steps, step, c["step"], c["tile"], partial)
+        if plan.ksplit > 1:
+            # the reduction reads ksplit partial tiles and writes C once
+            gpu += 2.5 + (plan.ksplit + 1) * esz * plan.Mp * plan.Np / 2.4e6
+    gpu = max(gpu, bytes_ / (0.7 * hw["hbm_bytes_per_s"]) * 1e6) + _pack_us(plan)
+    if plan.prec == FP8:
+        launches += 1          # the operands' largest magnitudes
+    return max(gpu, _CALL_US + _LAUNCH_US * (launches - 1)) * 1e-6, gpu * 1e-6
 
 
 def candidate_plans(pb: GettProblem, prec: int, groupM: int = 8) -> List[GettPlan]:
@@ -936,7 +1028,6 @@ def candidate_plans(pb: GettProblem, prec: int, groupM: int = 8) -> List[GettPla
             if pb.K <= bk:
                 plans.append(build_vector_plan(pb, prec, tile, groupM=groupM))
     plans += _packed_candidates(pb, prec, groupM)
-    # ties at the HBM floor are broken by the time the tile work alone would take
     plans.sort(key=lambda p: _estimate(p))
     return plans
 

@@ -267,3 +267,24 @@ def test_split_k_plans(seed):
             assert plan.ksplit == ks and plan.grid == 0
             out = emulate_split(plan, A, B, C, 0.75, 1.5)
             assert rel_frobenius(out, ref) < 1e-13, (sizes, ks)
+
+
+@pytest.mark.parametrize("pad", [1, 8, 64, 192, 1024])
+def test_plain_offsets_equal_the_coordinate_form(pad):
+    """Linearization.offsets() of a plain order (outer sums) against the general
+    coordinate form, for every index set and tensor of random contractions."""
+    from tccg_amd.plan import Linearization, _ext, _orders
+
+    from .random_cases import random_contraction as shuffled
+    for seed in range(24):
+        pb = shuffled(seed).problem
+        for labels in _orders(pb):
+            lin = Linearization.plain(labels, _ext(pb, labels))
+            coord, valid = lin.coords(pad)
+            for T in (pb.A, pb.B, pb.C):
+                want = np.zeros(coord.shape[0], dtype=np.int64)
+                for i, l in enumerate(lin.labels):
+                    want += coord[:, i] * max(0, T.stride_of_label(l))
+                want = np.where(valid, want, np.int64(INVALID)).astype(np.uint32)
+                got = lin.offsets(T, pad)
+                assert got.dtype == np.uint32 and np.array_equal(got, want)
