@@ -67,6 +67,7 @@ class Contraction:
         self._device_plans: Dict[Tuple, object] = {}
         self._tuned: Dict[int, GettPlan] = {}
         self._tuned_call: Dict[int, GettPlan] = {}
+        self._calls: Dict[object, object] = {}   # prec as given -> the device plan that calls use
 
     @classmethod
     def from_tccg(cls, text: str, fuse: bool = True) -> "Contraction":
@@ -118,6 +119,7 @@ class Contraction:
                                       candidates=split)[0], key=lambda m: m.seconds)
         self._tuned_call[p] = best.plan
         self._device_plans.pop((p, None, None), None)
+        self._calls.clear()
         return best
 
     def _call_plan(self, p: int) -> GettPlan:
@@ -141,7 +143,9 @@ class Contraction:
 
     def __call__(self, A, B, C, alpha: Optional[float] = None, beta: Optional[float] = None, prec="f32",
                  tile: Optional[int] = None, stream=None):
-        dp = self.device_plan(prec, tile)
+        dp = self._calls.get(prec) if tile is None else self.device_plan(prec, tile)
+        if dp is None:
+            dp = self._calls[prec] = self.device_plan(prec)
         dp.run(A, B, C, self.alpha if alpha is None else alpha, self.beta if beta is None else beta,
                stream=stream)
         return C

@@ -133,6 +133,23 @@ inline int resident_limit(const void* kern, int lds, int threads = 256) {
   return cus * per_cu;
 }
 
+// The same, looked up once per device and kernel (the two queries take longer
+// than the launch): `known` holds one entry per device id below kKnownDevices,
+// 0 until the first call there.
+constexpr int kKnownDevices = 64;
+struct ResidentLimits { std::atomic<int> cap[kKnownDevices] = {}; };
+inline int resident_limit(ResidentLimits& known, const void* kern, int lds, int threads = 256) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return 0;
+  if (dev >= kKnownDevices) return resident_limit(kern, lds, threads);
+  int cap = known.cap[dev].load(std::memory_order_relaxed);
+  if (cap == 0) {
+    cap = resident_limit(kern, lds, threads);
+    known.cap[dev].store(cap, std::memory_order_relaxed);
+  }
+  return cap;
+}
+
 template <int P, int BM, int BN, int BK, int WM, int WN, int MA, int MB, int WALK>
 int launch_kernel(const tccg::GettParams<typename tccg::PrecTraits<P>::TG>& prm, int grid, hipStream_t stream) {
   using S = tccg::TileShape<P, BM, BN, BK, WM, WN>;
@@ -144,7 +161,11 @@ int launch_kernel(const tccg::GettParams<typename tccg::PrecTraits<P>::TG>& prm,
   int lds = prm.kTiles == 1 ? S::LDS_BYTES / 2 : S::LDS_BYTES;
   if (WALK == 2) lds = (int)tccg::stream_lds_bytes<P, BM, BN, BK, WM, WN>(prm.tilesN);
   if (WALK != 0) {
-    const int cap = resident_limit(reinterpret_cast<const void*>(kern), lds);
+    // (the streaming walk's LDS depends on the problem, the persistent walk's
+    // only on whether it has a second stage)
+    static ResidentLimits known[2];
+    const int cap = WALK == 1 ? resident_limit(known[prm.kTiles == 1], reinterpret_cast<const void*>(kern), lds)
+                              : resident_limit(reinterpret_cast<const void*>(kern), lds);
     if (cap > 0 && grid > cap) grid = cap;
   }
   hipLaunchKernelGGL(kern, dim3(grid), dim3(256), lds, stream, prm);
@@ -365,7 +386,8 @@ int launch_packed_kernel(const tccg::GettParams<typename tccg::PrecTraits<P>::TG
   static std::atomic<uint64_t> lds_set{0};
   if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kern), SH::LDS_BYTES, lds_set)) return rc;
   if (PERSIST) {
-    const int cap = resident_limit(reinterpret_cast<const void*>(kern), SH::LDS_BYTES);
+    static ResidentLimits known;
+    const int cap = resident_limit(known, reinterpret_cast<const void*>(kern), SH::LDS_BYTES);
     if (cap > 0 && grid > cap) grid = cap;
   }
   hipLaunchKernelGGL(kern, dim3(grid), dim3(256), SH::LDS_BYTES, stream, prm);
@@ -422,7 +444,8 @@ int launch_packed_sw_kernel(const tccg::GettParams<float>& prm, int grid, hipStr
   auto kern = tccg::gett_packed_sw_kernel<P, BM, BN, BK, ST>;
   static std::atomic<uint64_t> lds_set{0};
   if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kern), SW::LDS_BYTES, lds_set)) return rc;
-  const int cap = resident_limit(reinterpret_cast<const void*>(kern), SW::LDS_BYTES, 512);
+  static ResidentLimits known;
+  const int cap = resident_limit(known, reinterpret_cast<const void*>(kern), SW::LDS_BYTES, 512);
   if (cap > 0 && grid > cap) grid = cap;
   const int nblocks = prm.tilesM * prm.tilesN;
   if (grid > nblocks) grid = nblocks;
