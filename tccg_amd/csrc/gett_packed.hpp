@@ -282,7 +282,7 @@ __device__ inline void store_tile_staged(const GettParams<typename PrecTraits<P>
           a = (e4 * VEC) % E0;
           b = (e4 * VEC) / E0;
         }
-        vec_t v = *reinterpret_cast<const vec_t*>(src + b * LD + a);
+        const vec_t v = *reinterpret_cast<const vec_t*>(src + b * LD + a);
         vec_t* g = reinterpret_cast<vec_t*>(dst + e4 * VEC);
         if (beta == TG(0)) {
           __builtin_nontemporal_store(alpha * v, g);
