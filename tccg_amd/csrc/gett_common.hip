@@ -33,10 +33,13 @@ __global__ void amax_kernel(const float* __restrict__ x, int64_t n, unsigned* ou
   }
 }
 
-// Blocks per operand of amax_pair_kernel at most: enough loads in flight for
-// the whole chip (1024 threads per CU), few enough that the last block reduces
-// their maxima in one load per thread.
-constexpr int kAmaxBlocks = 512;
+// Blocks per operand of amax_pair_kernel at most, and elements per block below
+// that: the blocks count themselves on one word, about 10 ns each, so there are
+// only as many as keep the chip's loads in flight (one per CU, four 16-byte
+// loads per thread).  2 x 5.3 MB: 648 blocks 12.2 us, 162 blocks 6.8 us;
+// 2 x 134 MB: 1024 blocks 46 us, 256 blocks 40 us.
+constexpr int kAmaxBlocks = 128;
+constexpr int kAmaxPerBlock = 16384;
 
 __device__ inline float block_max(float m, float* red) {
   for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_down(m, off, 64));
@@ -49,11 +52,12 @@ __device__ inline float block_max(float m, float* red) {
 
 // max|A| and max|B| in one launch: blocks [0, nbA) walk A, the rest B; each
 // stores its maximum, and the block that finishes last reduces them all, so
-// nothing has to be cleared beforehand.  What bounds it is latency, not bytes:
-// as two clears and two reductions (one atomic per block on the result word)
-// it took four launches and 26 us before the FP8 pack launch of 2 x 5.3 MB;
-// one launch takes 6 us.  Scratch: out[0..1], the count of finished blocks
-// (wraps to 0 by itself), then kAmaxBlocks maxima per operand.
+// nothing has to be cleared beforehand.  Latency bounds it, not the bytes.  The
+// maxima are stored and read device-coherently with a wait in place of release
+// and acquire fences, which write back and invalidate an L2 per block
+// (2 x 5.3 MB, 648 blocks: 18.5 us with fences, 13.4 us without).  Scratch:
+// out[0..1], the count of finished blocks (wraps to 0 by itself), then
+// kAmaxBlocks maxima per operand.
 __global__ void __launch_bounds__(256)
 amax_pair_kernel(const float* __restrict__ A, int64_t nA, const float* __restrict__ B, int64_t nB, int nbA,
                  float* out) {
@@ -72,21 +76,28 @@ amax_pair_kernel(const float* __restrict__ A, int64_t nA, const float* __restric
   const int64_t head = (4 - ((reinterpret_cast<uintptr_t>(x) >> 2) & 3)) & 3;
   const int64_t quads = n > head ? (n - head) / 4 : 0;
   const float4* q = reinterpret_cast<const float4*>(x + head);
-  for (int64_t i = first; i < quads; i += stride) {
-    const float4 v = q[i];
-    m = fmaxf(fmaxf(m, fmaxf(fabsf(v.x), fabsf(v.y))), fmaxf(fabsf(v.z), fabsf(v.w)));
+  auto max4 = [](float m, const float4& v) {
+    return fmaxf(fmaxf(m, fmaxf(fabsf(v.x), fabsf(v.y))), fmaxf(fabsf(v.z), fabsf(v.w)));
+  };
+  int64_t i = first;
+  for (; i + 3 * stride < quads; i += 4 * stride) {
+    const float4 v0 = q[i], v1 = q[i + stride], v2 = q[i + 2 * stride], v3 = q[i + 3 * stride];
+    m = max4(max4(max4(max4(m, v0), v1), v2), v3);
   }
+  for (; i < quads; i += stride) m = max4(m, q[i]);
   const int64_t rest = n - quads * 4;   // at most 6 elements, before and after the quads
   if (first < rest) m = fmaxf(m, fabsf(first < head ? x[first] : x[quads * 4 + first]));
   m = block_max(m, red);
   if (threadIdx.x == 0) {
     __hip_atomic_store(part + (second ? kAmaxBlocks : 0) + b, m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __threadfence();
+    // the device-coherent store has completed before the count
+    asm volatile("" ::: "memory");
+    tccg::wait_vm_lgkm0<0>();
+    asm volatile("" ::: "memory");
     last = atomicInc(done, gridDim.x - 1) == gridDim.x - 1;
   }
   __syncthreads();
   if (!last) return;
-  __threadfence();
   for (int op = 0; op < 2; ++op) {
     const int nb = op ? gridDim.x - nbA : nbA;
     float v = 0.f;
@@ -255,8 +266,7 @@ size_t tccg_amax_pair_floats(void) { return 4 + 2 * (size_t)tccg_lib::kAmaxBlock
 int tccg_amax_pair_f32(const float* A, int64_t nA, const float* B, int64_t nB, float* out, void* stream) {
   using namespace tccg_lib;
   if (!A || !B || !out || nA <= 0 || nB <= 0) return fail(1, "amax: bad arguments");
-  // 4096 elements (four 16-byte loads per thread) per block
-  auto blocks = [](int64_t n) { return (int)std::min<int64_t>((n + 4095) / 4096, kAmaxBlocks); };
+  auto blocks = [](int64_t n) { return (int)std::min<int64_t>((n + kAmaxPerBlock - 1) / kAmaxPerBlock, kAmaxBlocks); };
   const int nbA = blocks(nA), nbB = blocks(nB);
   hipLaunchKernelGGL(amax_pair_kernel, dim3(nbA + nbB), dim3(256), 0, (hipStream_t)stream, A, nA, B, nB, nbA, out);
   hipError_t e = hipGetLastError();
