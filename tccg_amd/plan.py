@@ -820,7 +820,7 @@ _GATHER_COST = {
     BF16: dict(mfma=8.6, step=0.80, tile=0.56, store=0.335, scalar=0.41, walk=0.0),
 }
 _CALL_US, _LAUNCH_US = 10.9, 2.9    # a call back to back with others: its first launch, every other one
-_PACK_US, _PACK_BW = 6.2, 4.5e12    # the pack launch with the gap after it; bytes/s it moves
+_PACK_US, _PACK_BW = 6.2, 4.5e12    # pack launch and the gap after it; bytes/s (large ones 5.8e12: same choices)
 
 
 def _c_segment_bytes(plan: GettPlan) -> float:
