@@ -792,9 +792,9 @@ def store_efficiency(segment_bytes: float) -> float:
 # plans near their contraction's best weighted up) to 17091 timed plans of 114
 # contractions: every pattern of tccg_amd.workloads over extents 8-72 (96-384
 # for the short-k pattern), every candidate plan.  The model's first choice
-# takes 1.04 (FP32), 1.02 (split-BF16), 1.04 (BF16), 1.04 (FP64) and 1.02 (FP8)
+# takes 1.035 (FP32), 1.02 (split-BF16), 1.04 (BF16), 1.03 (FP64) and 1.01 (FP8)
 # times the best candidate's time in the geometric mean, where the constants
-# before took 1.59, 1.42, 1.27, 1.15 and 1.06; the worst choice 1.95 times (5.2
+# before took 1.59, 1.42, 1.27, 1.15 and 1.06; the worst choice 1.53 times (5.2
 # before: store waves over a handful of tiles).
 #
 # Packed kernels, per precision: MFMA time of a k-step over the nominal peak
@@ -972,7 +972,7 @@ def _estimate(plan: GettPlan, beta: float = 0.0) -> Tuple[float, float]:
             if plan.crun[0]:   # the run epilogue's passes through LDS
                 partial = tile_store + 1.3 * store
             else:              # non-temporal stores, as above
-                partial = tile_store * (1.0 + 1.25 * (1.0 - _line_stores(plan)))
+                partial = tile_store * (1.0 + 1.8 * (1.0 - _line_stores(plan)))
         if plan.walk == 5:
             # the k-steps spread evenly over the grid; each workgroup walks
             # about a piece more than its share of tiles, and publishes and
@@ -993,7 +993,13 @@ def _estimate(plan: GettPlan, beta: float = 0.0) -> Tuple[float, float]:
         elif plan.grid:
             grid = max(1, min(plan.grid, cus * slots))
             j = max(1.0, grid / cus)
-            gpu = -(-n // grid) * (steps * max(c["step"], j * step) + 0.5 + 1.8 * j * tile_store) + c["tile"]
+            # a run of C that the tile's m range cuts is written as partial lines
+            # by two workgroups (FP8's fitted store time holds it); a workgroup
+            # alone on its CU has nothing to compute beside its stores
+            run = _leading_run(plan.offCm[:4096].astype(np.int64), 1)
+            cut = 1.0 + 3.0 * run / plan.BM if run < plan.BM and plan.prec != FP8 else 1.0
+            out = (1.3 * j if j > 1 else 2.2) * cut * tile_store
+            gpu = -(-n // grid) * (steps * max(c["step"], j * step) + 0.3 + out) + c["tile"]
         else:
             gpu = _rounds_us(n, slots, steps, step, c["step"], c["tile"], partial)
         if plan.ksplit > 1:
