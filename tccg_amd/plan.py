@@ -792,9 +792,9 @@ def store_efficiency(segment_bytes: float) -> float:
 # plans near their contraction's best weighted up) to 17091 timed plans of 114
 # contractions: every pattern of tccg_amd.workloads over extents 8-72 (96-384
 # for the short-k pattern), every candidate plan.  The model's first choice
-# takes 1.035 (FP32), 1.02 (split-BF16), 1.04 (BF16), 1.03 (FP64) and 1.01 (FP8)
+# takes 1.03 (FP32), 1.02 (split-BF16), 1.04 (BF16), 1.03 (FP64) and 1.01 (FP8)
 # times the best candidate's time in the geometric mean, where the constants
-# before took 1.59, 1.42, 1.27, 1.15 and 1.06; the worst choice 1.53 times (5.2
+# before took 1.59, 1.42, 1.27, 1.15 and 1.06; the worst choice 1.39 times (5.2
 # before: store waves over a handful of tiles).
 #
 # Packed kernels, per precision: MFMA time of a k-step over the nominal peak
@@ -960,9 +960,12 @@ def _estimate(plan: GettPlan, beta: float = 0.0) -> Tuple[float, float]:
             gpu = (-(-n // grid) * (steps * max(c["step"], j * step) + c["walk"] + 1.8 * j * c["store"] * store)
                    + c["tile"])
         else:
-            # non-temporal stores of partial lines go to HBM part by part
+            # non-temporal stores of partial lines go to HBM part by part, and
+            # of runs shorter than a store's lanes several times over (tiles
+            # over 64x64, whose stores queue up)
+            short = _c_segment_bytes(plan) < 128 and plan.BM * plan.BN > 64 * 64
             gpu = _rounds_us(n, slots, steps, step, c["step"], c["tile"],
-                             c["store"] * store * (1.0 + 1.2 * (1.0 - _line_stores(plan))))
+                             c["store"] * store * (1.0 + (2.0 if short else 1.2) * (1.0 - _line_stores(plan))))
     else:
         c = _PACKED_COST[plan.prec]
         launches = 3 if plan.ksplit > 1 else 2
@@ -972,7 +975,8 @@ def _estimate(plan: GettPlan, beta: float = 0.0) -> Tuple[float, float]:
             if plan.crun[0]:   # the run epilogue's passes through LDS
                 partial = tile_store + 1.3 * store
             else:              # non-temporal stores, as above
-                partial = tile_store * (1.0 + 1.8 * (1.0 - _line_stores(plan)))
+                short = _c_segment_bytes(plan) < 128 and plan.BM * plan.BN > 64 * 64
+                partial = tile_store * (1.0 + (3.0 if short else 1.8) * (1.0 - _line_stores(plan)))
         if plan.walk == 5:
             # the k-steps spread evenly over the grid; each workgroup walks
             # about a piece more than its share of tiles, and publishes and
@@ -1086,6 +1090,25 @@ def split_fits(plan: GettPlan) -> bool:
     return 3 * max(plan.Mp, plan.Np) * plan.Kp < 0xFFFFFF00
 
 
+def _chain(plan: GettPlan) -> float:
+    """k values that the plan adds up one after the other, at most (stream-k: a
+    segment, where the tiles are fewer than the workgroups)."""
+    n = plan.ntiles()
+    if plan.walk == 5 and n < plan.grid:
+        return min(plan.problem.K, plan.Kp * n / plan.grid)
+    return min(plan.problem.K, plan.Kp / plan.ksplit)
+
+
+def _chain_bound(pb: GettProblem) -> float:
+    """Longest summation chain of plans that calls in FP32 take: 1.3 times that
+    of FP32 stream-k over 128x128 tiles, which spreads k over the GPU where the
+    tiles are few.  The error grows with the chain's square root and the split's
+    is 0.87 times FP32's at equal chains, so no call is less exact than there
+    (one-tile split plans of 2401 x 221, k 3124: 7.6e-7 against 3.8e-7)."""
+    tiles = -(-pb.M // 128) * (-(-pb.N // 128))
+    return max(512.0, 1.3 * pb.K * min(1.0, tiles / MI355X["cus"]))
+
+
 def split_plans(pb: GettProblem, groupM: int = 8) -> List[GettPlan]:
     """Guarded split-BF16 packed plans for an FP32 contraction, best model
     estimate first: FP32 operands held exactly as three BF16 parts, the six
@@ -1096,6 +1119,8 @@ def split_plans(pb: GettProblem, groupM: int = 8) -> List[GettPlan]:
         return []
     plans = [p for p in _packed_candidates(pb, BF16X3, groupM)
              if p.walk in (0, 5) and p.ksplit == 1 and split_fits(p)]
+    bound = _chain_bound(pb)
+    plans = [p for p in plans if _chain(p) <= bound]
     for p in plans:
         p.guard = True
     plans.sort(key=lambda p: _estimate(p))
@@ -1107,6 +1132,8 @@ def call_plan(pb: GettProblem, prec: int) -> GettPlan:
     FP32 also the plans that compute it on the BF16 MFMAs."""
     best = default_plan(pb, prec)
     split = split_plans(pb)[:1] if prec == F32 else []
+    if split and _chain(best) > _chain_bound(pb):
+        return split[0]
     return min([best] + split, key=lambda p: _estimate(p))
 
 

@@ -107,3 +107,18 @@ def test_entry_rejects_what_it_cannot_run():
     cp.ksplit = 2
     assert lib.tccg_gett_f32_split(one, one, one, 1.0, 0.0, ctypes.byref(cp), one, 1 << 40, 0, None) != 0
     assert b"without ksplit" in lib.tccg_last_error()
+
+
+@pytest.mark.parametrize("m, n, k", [(221, 3124, 2401), (930, 840, 4002), (1239, 1936, 928), (5184, 5184, 2304),
+                                     (128, 128, 32), (64, 64, 20000), (300, 300, 511)])
+def test_calls_do_not_lengthen_the_summation_chains(m, n, k):
+    """FP32 calls add up at most 1.3 times the k values one after the other
+    that stream-k over 128x128 tiles would (512 where that is less)."""
+    from tccg_amd.plan import _chain
+    pb = Contraction.from_labels(["m", "n"], ["k", "m"], ["n", "k"], {"m": m, "n": n, "k": k}).problem
+    tiles = -(-m // 128) * -(-n // 128)
+    split = split_plans(pb)
+    if not split:                             # no split plan cuts k finely enough
+        assert call_plan(pb, F32).describe() == default_plan(pb, F32).describe()
+    for p in split and [call_plan(pb, F32)] + split:
+        assert _chain(p) <= max(512, 1.3 * k * min(1.0, tiles / 256)), p.describe()
