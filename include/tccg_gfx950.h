@@ -214,16 +214,16 @@ int tccg_gett_packed_fp8(const float* A, const float* B, float* C, float alpha, 
 /*
  * FP32 GETT on the BF16 MFMAs.  The packed split-BF16 kernels with FP32's
  * contract for every input: `plan` is a split-BF16 packed plan (walk 0 or 5,
- * no ksplit).  Where every value of a 64 x 32 pack block is 0 or has
- * 2^-100 <= |x| < 2^51 its three BF16 parts hold it exactly; a block with any
- * other value (infinities, NaNs, the extremes of the FP32 range) keeps its
- * FP32 bits, and the parts of C that read it are computed on the FP32 MFMA as
- * tccg_gett_packed_f32 computes them.  The workspace takes
- * tccg_f32_split_workspace_bytes().  prepacked != 0: the GETT kernel alone
- * over the operands of the previous call (A and B are not read).  The first
- * 4 bytes at the guard region are best cleared once when the workspace is
- * allocated (tccg_f32_split_clear_offset()): any other value there is
- * harmless, it only makes every tile look at its guard words.
+ * no ksplit).  Values below
+ * 2^((81 - log2 k) / 2) (2^34 at k = 4096), subnormals included, are held
+ * exactly by their three BF16 parts; a 64 x 32 pack block with any other value
+ * (larger ones, infinities, NaNs) keeps its FP32 bits, and the tiles of C that
+ * read it are computed on the FP32 MFMA, as tccg_gett_packed_f32 computes them.
+ * The workspace takes tccg_f32_split_workspace_bytes().  prepacked != 0: the
+ * GETT kernel alone over the operands of the previous call (A and B are not
+ * read).  The 16 bytes at tccg_f32_split_clear_offset() are best cleared once
+ * when the workspace is allocated: any other value there is harmless, it only
+ * makes the tiles of one call look at their guard words.
  */
 size_t tccg_f32_split_workspace_bytes(const tccg_gett_plan* plan);
 size_t tccg_f32_split_clear_offset(const tccg_gett_plan* plan);
@@ -358,7 +358,7 @@ int tccg_gett_group(int prec, int tile, const tccg_group_operand* ops, int nops,
 
 /* FP32 problems on the BF16 MFMAs, each with tccg_gett_f32_split's contract:
  * the records of a TCCG_BF16X3 group, with the first 256 bytes of the
- * workspace kept free (every `out` from 256 on; its first 4 bytes are best
+ * workspace kept free (every `out` from 256 on; its first 16 bytes are best
  * cleared once) and one guard word per 64 x 32 block of an operand
  * (fBlocks * kTiles * BK / 32 words) right after the operand's planes. */
 int tccg_gett_group_f32_split(int tile, const tccg_group_operand* ops, int nops, const tccg_group_job* jobs,

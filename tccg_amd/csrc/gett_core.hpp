@@ -51,7 +51,9 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef int i32x8 __attribute__((ext_vector_type(8)));
 
-enum Prec : int { F32 = 0, F64 = 1, BF16X3 = 2, FP8 = 3, BF16 = 4 };
+// F32X3 is internal: FP32 contractions through the three BF16 parts (the packed
+// kernels only; plans and callers name F32 or BF16X3).
+enum Prec : int { F32 = 0, F64 = 1, BF16X3 = 2, FP8 = 3, BF16 = 4, F32X3 = 5 };
 
 // How one operand's tile is gathered from HBM.  The host picks the mode from
 // where the operand's stride-one index sits:
@@ -107,11 +109,10 @@ struct GettParams {
   // word per workgroup (1: that workgroup's partial is complete) and, after
   // them, an error word (bit 0: a wait for a partial gave up).
   uint32_t* flags;
-  // FP32 through the split-BF16 kernels (packed walks of BF16X3, gett_packed.hpp):
-  // guardAny == nullptr for plain split-BF16, else a word that is nonzero when
-  // a 64 x 32 pack block may hold its values as raw FP32 bits, and one word per
-  // pack block of A and of B (row-block major, guardK blocks along k).
-  const uint32_t* guardAny = nullptr;
+  // FP32 through the split (F32X3, gett_packed.hpp): four words (guard_any(),
+  // gett_packed.hpp), and one word per 64 x 32 pack block of A and of B, nonzero
+  // where it holds raw FP32 bits (row-block major, guardK blocks along k).
+  uint32_t* guardAny = nullptr;
   const uint32_t* guardA = nullptr;
   const uint32_t* guardB = nullptr;
   int guardK = 0;
@@ -130,6 +131,7 @@ template <> struct PrecTraits<BF16X3> {
   using TG = float; using TL = __bf16;
   static constexpr int PLANES = 3, SUB = 32, KF = 16, PAD = 8, ACC = 16;
 };
+template <> struct PrecTraits<F32X3> : PrecTraits<BF16X3> {};
 template <> struct PrecTraits<BF16> {
   using TG = float; using TL = __bf16;
   static constexpr int PLANES = 1, SUB = 32, KF = 16, PAD = 8, ACC = 16;
@@ -413,6 +415,11 @@ template <> struct Mma<BF16X3> {
   }
 };
 
+// FP32 through the split.  The parts are those of the operand values times
+// kSplitScale (gett_pack.hpp split_limit()); the sums hold C times its square.
+constexpr float kSplitScale = 0x1p23f, kUnscale = 0x1p-46f;
+template <> struct Mma<F32X3> : Mma<BF16X3> {};
+
 template <> struct Mma<BF16> {
   using Frag = bf16x8;
   using Acc = f32x16;
@@ -526,15 +533,20 @@ __device__ inline void store_tile_from(const GettParams<typename PrecTraits<P>::
                                        typename Mma<P>::Acc (&acc)[TileShape<P, BM, BN, BK, WM, WN>::SN]
                                                                   [TileShape<P, BM, BN, BK, WM, WN>::SM],
                                        const uint32_t* cmT, const uint32_t* cnT, int wm, int wn, int lane,
-                                       float descale, bool checker = false) {
+                                       float descale) {
   using TR = PrecTraits<P>;
   using TG = typename TR::TG;
   using S = TileShape<P, BM, BN, BK, WM, WN>;
   using MM = Mma<P>;
-  // alpha by the parity of n (that of the accumulator register); checker: the
-  // accumulators hold (-1)^(m + n) C (m's parity is the lane's, pack_block)
-  const TG beta = p.beta;
-  const TG alpha[2] = {checker && (lane & 1) ? -p.alpha : p.alpha, checker && !(lane & 1) ? -p.alpha : p.alpha};
+  // F32X3: the accumulators hold (-1)^(m + n) C over `descale` (pack_block); m's
+  // parity is the lane's, n's that of the accumulator register.
+  const TG alpha = p.alpha, beta = p.beta;
+  const float sign[2] = {lane & 1 ? -descale : descale, lane & 1 ? descale : -descale};
+  auto value = [&](const typename MM::Acc& a, int r) {
+    if constexpr (P == F32X3) return sign[r & 1] * a[r];
+    else if constexpr (P == FP8) return (TG)((float)a[r] * descale);
+    else return (TG)a[r];
+  };
   uint32_t cm[S::SM], cn[S::SN][MM::NACC];
 #pragma unroll
   for (int j = 0; j < S::SM; ++j) {
@@ -569,11 +581,10 @@ __device__ inline void store_tile_from(const GettParams<typename PrecTraits<P>::
       for (int r = 0; r < MM::NACC; ++r)
 #pragma unroll
         for (int j = 0; j < S::SM; ++j) {
-          TG val = (TG)acc[i][j][r];
-          if (P == FP8) val = (TG)((float)val * descale);
+          const TG val = value(acc[i][j], r);
           TG* dst = p.C + (size_t)(cm[j] + cn[i][r]);
-          if constexpr (WB) *dst = alpha[r & 1] * val;
-          else __builtin_nontemporal_store(alpha[r & 1] * val, dst);
+          if constexpr (WB) *dst = alpha * val;
+          else __builtin_nontemporal_store(alpha * val, dst);
         }
     return;
   }
@@ -586,11 +597,10 @@ __device__ inline void store_tile_from(const GettParams<typename PrecTraits<P>::
 #pragma unroll
         for (int j = 0; j < S::SM; ++j)
           if (cm[j] != kInvalid && cn[i][r] != kInvalid) {
-            TG val = (TG)acc[i][j][r];
-            if (P == FP8) val = (TG)((float)val * descale);
+            const TG val = value(acc[i][j], r);
             TG* dst = p.C + (size_t)(cm[j] + cn[i][r]);
-            if constexpr (WB) *dst = alpha[r & 1] * val;
-            else __builtin_nontemporal_store(alpha[r & 1] * val, dst);
+            if constexpr (WB) *dst = alpha * val;
+            else __builtin_nontemporal_store(alpha * val, dst);
           }
     return;
   }
@@ -619,9 +629,8 @@ __device__ inline void store_tile_from(const GettParams<typename PrecTraits<P>::
 #pragma unroll
         for (int j = 0; j < S::SM; ++j)
           if (cm[j] != kInvalid && cn[i][r0 + r] != kInvalid) {
-            TG val = (TG)acc[i][j][r0 + r];
-            if (P == FP8) val = (TG)((float)val * descale);
-            p.C[(size_t)(cm[j] + cn[i][r0 + r])] = alpha[(r0 + r) & 1] * val + beta * c[r][j];
+            const TG val = value(acc[i][j], r0 + r);
+            p.C[(size_t)(cm[j] + cn[i][r0 + r])] = alpha * val + beta * c[r][j];
           }
     }
 }
@@ -630,8 +639,8 @@ template <int P, int BM, int BN, int BK, int WM, int WN, bool DRAIN = false>
 __device__ inline void store_tile(const GettParams<typename PrecTraits<P>::TG>& p,
                                   typename Mma<P>::Acc (&acc)[TileShape<P, BM, BN, BK, WM, WN>::SN]
                                                              [TileShape<P, BM, BN, BK, WM, WN>::SM],
-                                  int m0, int n0, int wm, int wn, int lane, float descale, bool checker = false) {
-  store_tile_from<P, BM, BN, BK, WM, WN, DRAIN>(p, acc, p.offCm + m0, p.offCn + n0, wm, wn, lane, descale, checker);
+                                  int m0, int n0, int wm, int wn, int lane, float descale) {
+  store_tile_from<P, BM, BN, BK, WM, WN, DRAIN>(p, acc, p.offCm + m0, p.offCn + n0, wm, wn, lane, descale);
 }
 
 // One BM x BN tile (tm, tn) of C over the whole k range, computed by the 256

@@ -8,19 +8,20 @@ namespace tccg {
 
 // One 64 x 32 block per workgroup: job blockIdx.x of the list.
 //
-// guard (BF16X3: FP32 through the split, gett_pack.hpp): an operand's guard
-// words follow its planes, the word that any raw block sets begins the
-// workspace.
+// F32X3 (FP32 through the split, gett_pack.hpp): an operand's guard words follow
+// its planes, guard_any()'s words begin the workspace.
 template <int P, int BM, int BN, int BK>
 __global__ void __launch_bounds__(256)
 group_pack_kernel(const tccg_group_operand* __restrict__ ops, int nops, const tccg_group_job* __restrict__ jobs,
-                  int njobs, unsigned char* ws, size_t ws_bytes, int guard) {
+                  int njobs, unsigned char* ws, size_t ws_bytes) {
+  constexpr bool guard = P == F32X3;
   using TR = PrecTraits<P>;
   using TG = typename TR::TG;
   using TL = typename TR::TL;
   __shared__ TG tile[kPackTF][kPackTK + 1];
   const int j = blockIdx.x;
   if (j >= njobs) return;
+  if (guard && j == 0 && threadIdx.x == 0) guard_pack_turn(reinterpret_cast<uint32_t*>(ws));
   const tccg_group_job jb = jobs[j];
   if (jb.item < 0 || jb.item >= nops) return;
   const tccg_group_operand& op = ops[jb.item];
@@ -49,7 +50,8 @@ group_pack_kernel(const tccg_group_operand* __restrict__ ops, int nops, const tc
 template <int P, int BM, int BN, int BK, int WM, int WN, int S>
 __global__ void __launch_bounds__(256)
 gett_group_kernel(const tccg_group_problem* __restrict__ probs, int nprobs, const tccg_batch_work* __restrict__ work,
-                  int nwork, const unsigned char* __restrict__ ws, size_t ws_bytes, int guard) {
+                  int nwork, unsigned char* ws, size_t ws_bytes) {
+  constexpr bool guard = P == F32X3;
   using TR = PrecTraits<P>;
   using TG = typename TR::TG;
   using SH = PackedShape<P, BM, BN, BK, S>;
@@ -79,11 +81,17 @@ gett_group_kernel(const tccg_group_problem* __restrict__ probs, int nprobs, cons
   p.alpha = (TG)q.alpha; p.beta = (TG)q.beta;
   p.amax = nullptr;
   p.crunM = 0; p.crunN = 0; p.cvec = 0; p.ksplit = 1; p.part = nullptr; p.flags = nullptr;
-  if (guard) {
-    p.guardAny = reinterpret_cast<const uint32_t*>(ws);
+  if constexpr (guard) {
+    p.guardAny = reinterpret_cast<uint32_t*>(ws);
     p.guardA = reinterpret_cast<const uint32_t*>(ws + q.packedA + pa);
     p.guardB = reinterpret_cast<const uint32_t*>(ws + q.packedB + pb);
     p.guardK = nK;
+  }
+  if constexpr (guard) {
+    const bool any = guard_any(p, v == 0 && threadIdx.x == 0);
+    if (const int raw = any ? tile_raw<BM, BN>(p, wk.tm, wk.tn) : 0)
+      return packed_walk<P, BM, BN, BK, WM, WN, S, false, false, true>(p, v, nwork, wk.tm, wk.tn, 0, 0, q.kTiles,
+                                                                       smem_raw, SkPiece{}, raw);
   }
   packed_walk<P, BM, BN, BK, WM, WN, S, false>(p, v, nwork, wk.tm, wk.tn, 0, 0, q.kTiles, smem_raw);
 }
@@ -95,20 +103,19 @@ namespace tccg_lib {
 template <int P, int I = 0>
 int launch_group(int tile, const tccg_group_operand* ops, int nops, const tccg_group_job* jobs, int njobs,
                  const tccg_group_problem* probs, int nprobs, const tccg_batch_work* work, int nwork, void* ws,
-                 size_t ws_bytes, int guard, hipStream_t s) {
+                 size_t ws_bytes, hipStream_t s) {
   if constexpr (I >= packed_count(P)) {
     return fail(1, "invalid packed tile id");
   } else {
     constexpr TileCfg c = packed_tile(P, I);
     if (tile != I)
-      return launch_group<P, I + 1>(tile, ops, nops, jobs, njobs, probs, nprobs, work, nwork, ws, ws_bytes, guard,
-                                    s);
+      return launch_group<P, I + 1>(tile, ops, nops, jobs, njobs, probs, nprobs, work, nwork, ws, ws_bytes, s);
     constexpr int ST = kPackedStages;
     using SH = tccg::PackedShape<P, c.BM, c.BN, c.BK, ST>;
     unsigned char* wsb = reinterpret_cast<unsigned char*>(ws);
     if (njobs > 0) {
       hipLaunchKernelGGL((tccg::group_pack_kernel<P, c.BM, c.BN, c.BK>), dim3(njobs), dim3(256), 0, s, ops, nops,
-                         jobs, njobs, wsb, ws_bytes, guard);
+                         jobs, njobs, wsb, ws_bytes);
       hipError_t e = hipGetLastError();
       if (e != hipSuccess) return fail((int)e, std::string("group pack launch: ") + hipGetErrorString(e));
     }
@@ -117,7 +124,7 @@ int launch_group(int tile, const tccg_group_operand* ops, int nops, const tccg_g
       static std::atomic<uint64_t> lds_set{0};
       if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kern), SH::LDS_BYTES, lds_set)) return rc;
       hipLaunchKernelGGL(kern, dim3(nwork), dim3(256), SH::LDS_BYTES, s, probs, nprobs, work, nwork,
-                         (const unsigned char*)wsb, ws_bytes, guard);
+                         wsb, ws_bytes);
       hipError_t e = hipGetLastError();
       if (e != hipSuccess) return fail((int)e, std::string("group GETT launch: ") + hipGetErrorString(e));
     }
@@ -128,7 +135,7 @@ int launch_group(int tile, const tccg_group_operand* ops, int nops, const tccg_g
 template <int P>
 int run_group(int tile, const tccg_group_operand* ops, int nops, const tccg_group_job* jobs, int njobs,
               const tccg_group_problem* probs, int nprobs, const tccg_batch_work* work, int nwork, void* ws,
-              size_t ws_bytes, void* stream, int guard = 0) {
+              size_t ws_bytes, void* stream) {
   if (nops < 0 || njobs < 0 || nprobs < 0 || nwork < 0) return fail(1, "negative count");
   if ((njobs > 0 && (!ops || !jobs || nops == 0)) || (nwork > 0 && (!probs || !work || nprobs == 0)))
     return fail(1, "group array is NULL or empty");
@@ -138,7 +145,7 @@ int run_group(int tile, const tccg_group_operand* ops, int nops, const tccg_grou
   packed_tiles_of(P, &ntiles);
   if (tile < 0 || tile >= ntiles) return fail(1, "invalid packed tile id");
   return launch_group<P>(tile, ops, nops, jobs, njobs, probs, nprobs, work, nwork, ws, ws_bytes,
-                         guard, (hipStream_t)stream);
+                         (hipStream_t)stream);
 }
 
 }  // namespace tccg_lib

@@ -87,7 +87,7 @@ inline const TileCfg* vector_tiles_of(int prec, int* n) {
 constexpr int packed_count(int prec) {
   return prec == tccg::F32 ? (int)(sizeof(kF32PackedTiles) / sizeof(TileCfg))
        : prec == tccg::F64 ? (int)(sizeof(kF64PackedTiles) / sizeof(TileCfg))
-       : prec == tccg::BF16X3 ? (int)(sizeof(kBfPackedTiles) / sizeof(TileCfg))
+       : prec == tccg::BF16X3 || prec == tccg::F32X3 ? (int)(sizeof(kBfPackedTiles) / sizeof(TileCfg))
        : prec == tccg::FP8 ? (int)(sizeof(kF8PackedTiles) / sizeof(TileCfg))
        : prec == tccg::BF16 ? (int)(sizeof(kBf1PackedTiles) / sizeof(TileCfg)) : 0;
 }
@@ -95,7 +95,7 @@ constexpr int packed_count(int prec) {
 constexpr TileCfg packed_tile(int prec, int i) {
   return prec == tccg::F32 ? kF32PackedTiles[i]
        : prec == tccg::F64 ? kF64PackedTiles[i]
-       : prec == tccg::BF16X3 ? kBfPackedTiles[i]
+       : prec == tccg::BF16X3 || prec == tccg::F32X3 ? kBfPackedTiles[i]
        : prec == tccg::FP8 ? kF8PackedTiles[i] : kBf1PackedTiles[i];
 }
 
@@ -103,7 +103,8 @@ inline const TileCfg* packed_tiles_of(int prec, int* n) {
   switch (prec) {
     case tccg::F32: *n = (int)(sizeof(kF32PackedTiles) / sizeof(TileCfg)); return kF32PackedTiles;
     case tccg::F64: *n = (int)(sizeof(kF64PackedTiles) / sizeof(TileCfg)); return kF64PackedTiles;
-    case tccg::BF16X3: *n = (int)(sizeof(kBfPackedTiles) / sizeof(TileCfg)); return kBfPackedTiles;
+    case tccg::BF16X3:
+    case tccg::F32X3: *n = (int)(sizeof(kBfPackedTiles) / sizeof(TileCfg)); return kBfPackedTiles;
     case tccg::FP8: *n = (int)(sizeof(kF8PackedTiles) / sizeof(TileCfg)); return kF8PackedTiles;
     case tccg::BF16: *n = (int)(sizeof(kBf1PackedTiles) / sizeof(TileCfg)); return kBf1PackedTiles;
     default: *n = 0; return nullptr;
@@ -338,7 +339,8 @@ inline size_t packed_workspace_bytes(int prec, const tccg_gett_plan* plan, size_
   size_t esz = 4, planes = 1;
   switch (prec) {
     case tccg::F64: esz = 8; break;
-    case tccg::BF16X3: esz = 2; planes = 3; break;
+    case tccg::BF16X3:
+    case tccg::F32X3: esz = 2; planes = 3; break;
     case tccg::BF16: esz = 2; break;
     case tccg::FP8: esz = 1; break;
     default: break;
@@ -365,7 +367,7 @@ inline size_t packed_workspace_bytes(int prec, const tccg_gett_plan* plan, size_
 // word that any raw pack block sets, padded to 256 bytes, and one guard word
 // per 64 x 32 pack block of A and of B.  0 if the plan is no packed plan.
 inline size_t f32_split_workspace_bytes(const tccg_gett_plan* plan, size_t* offG = nullptr) {
-  const size_t base = packed_workspace_bytes(tccg::BF16X3, plan, nullptr);
+  const size_t base = packed_workspace_bytes(tccg::F32X3, plan, nullptr);
   if (base == 0) return 0;
   const size_t g = (base - tccg::kPackedTailBytes + 255) & ~(size_t)255;
   const size_t words = ((size_t)plan->Mp / tccg::kPackTF + (size_t)plan->Np / tccg::kPackTF) *
@@ -533,7 +535,7 @@ int dispatch_packed_tile(int tile, const tccg::GettParams<typename tccg::PrecTra
         if (grid > 0 && grid < nblocks) return fail(1, "the run epilogue is built for one tile per workgroup");
       }
       if (grid > 0 && grid < nblocks) return launch_packed_kernel<P, c.BM, c.BN, c.BK, c.WM, c.WN, true>(prm, grid, s);
-      if (prm.ksplit > 1) {
+      if (P != tccg::F32X3 && prm.ksplit > 1) {
         // (k part, tile) work items, then the reduction of the parts into C
         int rc = launch_packed_kernel<P, c.BM, c.BN, c.BK, c.WM, c.WN, false>(prm, nblocks * prm.ksplit, s);
         if (rc) return rc;
@@ -602,13 +604,14 @@ int pack_operands(int tile, const typename tccg::PrecTraits<P>::TG* A, const typ
 // pack == true: pack A and B into the workspace, then the GETT kernel;
 // pack == false: the GETT kernel alone over operands a previous call with
 // the same plan and workspace has packed (A and B are not read).
-// guard (BF16X3): FP32 results, pack blocks that the split does not hold kept
-// as raw FP32 values and their tiles computed on the FP32 MFMA.
+// F32X3: pack blocks that the split does not hold are kept as raw FP32 values,
+// and the k-steps that read them run on the FP32 MFMA.
 template <int P>
 int run_gett_packed(const typename tccg::PrecTraits<P>::TG* A, const typename tccg::PrecTraits<P>::TG* B,
                     typename tccg::PrecTraits<P>::TG* C, typename tccg::PrecTraits<P>::TG alpha,
                     typename tccg::PrecTraits<P>::TG beta, const tccg_gett_plan* plan, void* workspace,
-                    size_t workspace_bytes, void* stream, bool pack = true, bool guard = false) {
+                    size_t workspace_bytes, void* stream, bool pack = true) {
+  constexpr bool guard = P == tccg::F32X3;
   using TG = typename tccg::PrecTraits<P>::TG;
   using TL = typename tccg::PrecTraits<P>::TL;
   if (!plan) return fail(1, "plan is NULL");
@@ -662,7 +665,6 @@ int run_gett_packed(const typename tccg::PrecTraits<P>::TG* A, const typename tc
                               : nullptr;
   uint32_t* any = nullptr;
   if (guard) {
-    if (P != tccg::BF16X3) return fail(1, "FP32 through the split takes split-BF16 plans");
     if ((plan->walk != 0 && plan->walk != 5) || plan->ksplit > 1)
       return fail(1, "FP32 through the split takes packed plans of walk 0 or 5 without ksplit");
     any = reinterpret_cast<uint32_t*>(reinterpret_cast<unsigned char*>(workspace) + offG);
@@ -708,7 +710,7 @@ int run_gett_packed(const typename tccg::PrecTraits<P>::TG* A, const typename tc
     if (rc) return rc;
   }
   if (plan->walk == 4) {
-    if constexpr (std::is_same<TG, float>::value) return dispatch_packed_sw_tile<P>(plan->tile, prm, plan->grid, s);
+    if constexpr (std::is_same<TG, float>::value && !guard) return dispatch_packed_sw_tile<P>(plan->tile, prm, plan->grid, s);
   }
   if (plan->walk == 5) return dispatch_packed_sk_tile<P>(plan->tile, prm, plan->grid, s);
   return dispatch_packed_tile<P>(plan->tile, prm, plan->grid, s);

@@ -72,6 +72,7 @@ template <> struct PackWriter<BF16X3> {
     *reinterpret_cast<bf16x8*>(dst + 2 * plane_stride) = p2;
   }
 };
+template <> struct PackWriter<F32X3> : PackWriter<BF16X3> {};
 template <> struct PackWriter<BF16> {
   __device__ static inline void write8(__bf16* blk, int F, int, int r, int kin, const float* v, float) {
     bf16x8 p0;
@@ -95,19 +96,22 @@ template <> struct PackWriter<FP8> {
   }
 };
 
-// FP32 through the split: a value's three BF16 parts represent it exactly, and
-// the six products of two such values differ from the FP32 product by less
-// than FP32's own rounding, while every part stays a normal BF16 number and no
-// product or sum of the parts can overflow before the FP32 one does.  That
-// holds for 0 and for 2^-100 <= |x| < 2^51; infinities, NaNs and the extremes
-// of the FP32 range do not qualify.
-__device__ inline bool split_holds(float x) {
-  const uint32_t u = __float_as_uint(x);
-  return (u << 1) == 0u || ((u >> 23) & 0xffu) - 27u <= 150u;
+// FP32 through the split (F32X3): the parts are taken of x 2^23 (kSplitScale).
+// The lowest bit of any FP32 number is 2^-149 or more, that of x 2^23 so 2^-126
+// or more: for numbers of every size, subnormals included, the three parts are
+// zero or normal BF16 numbers and add up to x 2^23 exactly.  What bounds a held
+// value is that no sum may overflow: with |x| < 2^h in both operands, k products
+// add up to less than k 2^(2 h + 46) <= 2^127 for h = (81 - log2 k) / 2, rounded
+// down (2^34 at k = 4096).  Larger values, infinities and NaNs are not held.
+// Returns the FP32 bits of 2^h.
+__device__ inline uint32_t split_limit(int Kp) {
+  const int h = (81 - (32 - __builtin_clz((unsigned)Kp - 1u))) / 2;
+  return (uint32_t)(127 + h) << 23;
 }
+__device__ inline bool split_holds(float x, uint32_t limit) { return (__float_as_uint(x) & 0x7fffffffu) < limit; }
 
 // The same eight values as their FP32 bits: high halves in plane 0, low halves
-// in plane 1 (plane 2 is not read for such a block).
+// in plane 1, the mark in plane 2.
 __device__ inline void write8_raw(__bf16* blk, int F, int plane_stride, int r, int kin, const float* v) {
   typedef unsigned short u16x8 __attribute__((ext_vector_type(8)));
   u16x8 hi, lo;
@@ -120,7 +124,7 @@ __device__ inline void write8_raw(__bf16* blk, int F, int plane_stride, int r, i
   __bf16* dst = blk + chunk_pos<__bf16>(F, r, kin >> 3);
   *reinterpret_cast<u16x8*>(dst) = hi;
   *reinterpret_cast<u16x8*>(dst + plane_stride) = lo;
-  *reinterpret_cast<u16x8*>(dst + 2 * plane_stride) = u16x8{};
+  *reinterpret_cast<u16x8*>(dst + 2 * plane_stride) = u16x8{} + kRawMark;
 }
 
 constexpr int kPackTF = 64;  // free positions per pack workgroup
@@ -170,10 +174,9 @@ struct PackGroup {
 // The 64 x 32 block at free position f0, k position k0 (tile: the
 // workgroup's LDS staging buffer).
 //
-// guard (BF16X3 only, nullptr otherwise): this block's guard word.  A block
-// with a value outside split_holds() keeps all of its values as raw FP32 bits
-// and sets its word and `any`; every other block clears its word.  `any` is
-// never cleared here: once set it only makes the GETT kernel look at the words.
+// guard (F32X3 only): this block's guard word.  A block with a value outside
+// split_holds() keeps all of its values as raw FP32 bits and sets its word and
+// this call's word of `any` (guard_any()); every other block clears its word.
 // Odd rows are stored negated, in both operands, so that the accumulator of
 // C(m, n) holds (-1)^(m + n) C(m, n), which the epilogue undoes.  The BF16 MFMA
 // cuts its aligned addends off towards minus infinity (measured: about 1/600 of
@@ -241,25 +244,25 @@ __device__ __forceinline__ void pack_block(const typename PrecTraits<P>::TG* __r
   }
   const int gf = f0 + f, gk = k0 + kl;
   const size_t blk = (size_t)(gf / F) * (size_t)kTiles * BLOCK + (size_t)(gk / BK) * BLOCK;
-  if constexpr (P == BF16X3) {
-    if (guard) {
-      if (f & 1) {
+  if constexpr (P == F32X3) {
+    const uint32_t limit = split_limit(kTiles * BK);
+    bool bad = false;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = -v[j];
-      }
-      bool bad = false;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) bad = bad || !split_holds(v[j]);
-      const int raw = __syncthreads_or(bad);
-      if (t == 0) {
-        *guard = raw ? 1u : 0u;
-        if (raw) *any = 1u;
-      }
-      if (raw) {
-        write8_raw(out + blk, F, F * BK, gf % F, gk % BK, v);
-        return;
-      }
+    for (int j = 0; j < 8; ++j) {
+      bad = bad || !split_holds(v[j], limit);
+      v[j] = f & 1 ? -v[j] : v[j];
     }
+    const int raw = __syncthreads_or(bad);
+    if (t == 0) {
+      *guard = raw ? 1u : 0u;
+      if (raw) any[any[2] & 1u] = 1u;
+    }
+    if (raw) {
+      write8_raw(out + blk, F, F * BK, gf % F, gk % BK, v);
+      return;
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] *= kSplitScale;
   }
   PackWriter<P>::write8(out + blk, F, F * BK, gf % F, gk % BK, v, scale);
 }
@@ -285,11 +288,18 @@ struct PackPair {
   int kTiles;
   uint32_t* clear;
   int nclear;
-  // FP32 through the split (BF16X3): a word per pack block of each operand
-  // (index (f0 / 64) * nK + k0 / 32) and the word that any raw block sets
+  // FP32 through the split (F32X3): a word per pack block of each operand
+  // (index (f0 / 64) * nK + k0 / 32) and the words of guard_any()
   uint32_t* guard[2] = {nullptr, nullptr};
   uint32_t* any = nullptr;
 };
+
+// The pack launch's part of guard_any()'s words (any one thread of it).
+__device__ inline void guard_pack_turn(uint32_t* any) {
+  const uint32_t turn = any[2] & 1u;
+  any[3] = turn;
+  any[turn ^ 1u] = 0u;
+}
 
 template <int P, int FA, int FB, int BK>
 __global__ void __launch_bounds__(256)
@@ -297,6 +307,7 @@ pack_pair_kernel(PackPair<typename PrecTraits<P>::TG, typename PrecTraits<P>::TL
   __shared__ typename PrecTraits<P>::TG tile[kPackTF][kPackTK + 1];
   if (blockIdx.x == 0)
     for (int i = threadIdx.x; i < q.nclear; i += 256) q.clear[i] = 0u;
+  if (P == F32X3 && blockIdx.x == 0 && threadIdx.x == 0) guard_pack_turn(q.any);
   const int nA = q.nF[0] * q.nK;
   int lb = xcd_chunked(blockIdx.x, gridDim.x);
   const int op = lb < nA ? 0 : 1;

@@ -60,6 +60,29 @@ __device__ inline void step_sync() {
   __builtin_amdgcn_sched_barrier(0);
 }
 
+// Issue order inside a k-step of NM MFMAs: the next step's NREAD LDS reads one
+// after each of the first MFMAs, then the NCOPY copies one after each of the
+// following, then the remaining MFMAs.
+template <int NM, int NREAD, int NCOPY>
+__device__ inline void step_schedule() {
+  constexpr int NR = NREAD < NM ? NREAD : NM;
+  constexpr int LEFT = NM - NR;
+  constexpr int NV = NCOPY < LEFT ? NCOPY : LEFT;
+#pragma unroll
+  for (int i = 0; i < NR; ++i) {
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+  }
+  __builtin_amdgcn_sched_group_barrier(0x100, NREAD - NR, 0);
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+  }
+  __builtin_amdgcn_sched_group_barrier(0x020, NCOPY - NV, 0);
+  __builtin_amdgcn_sched_group_barrier(0x008, LEFT - NV, 0);
+}
+
 template <int P, int BM, int BN, int BK, int S>
 struct PackedShape {
   using TR = PrecTraits<P>;
@@ -128,7 +151,7 @@ template <> struct PackedRead<FP8> {
 template <int P, int F, int BK>
 __device__ inline typename Mma<P>::Frag packed_frag(const typename PrecTraits<P>::TL* base, int row0, int kk,
                                                     int lane) {
-  if constexpr (P == BF16X3) return PackedRead<P>::read3(base, F, F * BK, row0, kk, lane);
+  if constexpr (P == BF16X3 || P == F32X3) return PackedRead<BF16X3>::read3(base, F, F * BK, row0, kk, lane);
   else return PackedRead<P>::read(base, F, row0, kk, lane);
 }
 
@@ -186,21 +209,59 @@ struct PackedCopier {
   }
 };
 
+// F32X3: the fragments of blocks held as raw FP32 bits (gett_pack.hpp
+// write8_raw) carry this in plane 2, where a held value's third part, a finite
+// number, never has it.
+constexpr unsigned short kRawMark = 0xffffu;
+
+// Whether a wave's fragment (32 rows of one pack block) holds raw bits.
+__device__ inline bool frag_raw(const Bf16x3Frag& f) {
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+  return __builtin_amdgcn_readfirstlane(__builtin_bit_cast(u32x4, f.p[2])[0]) == (uint32_t)kRawMark * 0x10001u;
+}
+
+// The eight values of a fragment: their raw FP32 bits, or the sums of the three
+// parts (exact: they do not overlap) without kSplitScale.
+__device__ inline void frag_values(const Bf16x3Frag& f, float (&v)[8]) {
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+  const u32x4 h = __builtin_bit_cast(u32x4, f.p[0]), m = __builtin_bit_cast(u32x4, f.p[1]),
+              l = __builtin_bit_cast(u32x4, f.p[2]);
+  if (frag_raw(f)) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      v[2 * i] = __uint_as_float(__builtin_amdgcn_perm(h[i], m[i], 0x05040100u));
+      v[2 * i + 1] = __uint_as_float(__builtin_amdgcn_perm(h[i], m[i], 0x07060302u));
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      v[2 * i] = (__uint_as_float(h[i] << 16) + (__uint_as_float(m[i] << 16) + __uint_as_float(l[i] << 16))) *
+                 (1.f / kSplitScale);
+      v[2 * i + 1] = (__uint_as_float(h[i] & 0xffff0000u) +
+                      (__uint_as_float(m[i] & 0xffff0000u) + __uint_as_float(l[i] & 0xffff0000u))) *
+                     (1.f / kSplitScale);
+    }
+  }
+}
+
 // Fragments of one k-step for this wave (all k sub-steps of the step).
 template <int P, int BM, int BN, int BK, int WM, int WN>
 struct PackedFrags {
   using TS = TileShape<P, BM, BN, BK, WM, WN>;
   static constexpr int NKK = BK / PrecTraits<P>::KF;
   // LDS reads and MFMA instructions per k-step of one wave
-  static constexpr int NREAD = NKK * (TS::SM + TS::SN) * (P == BF16X3 ? 3 : P == FP8 ? 2 : 1);
+  static constexpr int NREAD = NKK * (TS::SM + TS::SN) * (PrecTraits<P>::PLANES == 3 ? 3 : P == FP8 ? 2 : 1);
   static constexpr int NMFMA = NKK * TS::SM * TS::SN * Mma<P>::PARTS;
   typename Mma<P>::Frag a[NKK][TS::SM], b[NKK][TS::SN];
 
   __device__ inline void read(const unsigned char* stage, int wm, int wn, int lane) {
+    read(stage, stage + PackedShape<P, BM, BN, BK, 3>::BYTES_A, wm, wn, lane);
+  }
+  // from the block of A and that of B
+  __device__ inline void read(const unsigned char* blkA, const unsigned char* blkB, int wm, int wn, int lane) {
     using TL = typename PrecTraits<P>::TL;
-    using SH = PackedShape<P, BM, BN, BK, 3>;
-    const TL* As = reinterpret_cast<const TL*>(stage);
-    const TL* Bs = reinterpret_cast<const TL*>(stage + SH::BYTES_A);
+    const TL* As = reinterpret_cast<const TL*>(blkA);
+    const TL* Bs = reinterpret_cast<const TL*>(blkB);
 #pragma unroll
     for (int q = 0; q < NKK; ++q) {
 #pragma unroll
@@ -224,6 +285,53 @@ struct PackedFrags {
 #pragma unroll
           for (int j = 0; j < TS::SM; ++j) Mma<P>::mma_part(acc[i][j], b[q][i], a[q][j], part);
   }
+
+  // F32X3: whether any of the fragments holds raw FP32 bits.
+  __device__ inline bool raw() const {
+    bool r = false;
+#pragma unroll
+    for (int q = 0; q < NKK; ++q) {
+#pragma unroll
+      for (int j = 0; j < TS::SM; ++j) r = r || frag_raw(a[q][j]);
+#pragma unroll
+      for (int i = 0; i < TS::SN; ++i) r = r || frag_raw(b[q][i]);
+    }
+    return r;
+  }
+
+  __device__ inline void clear() {
+#pragma unroll
+    for (int q = 0; q < NKK; ++q) {
+#pragma unroll
+      for (int j = 0; j < TS::SM; ++j) a[q][j] = typename Mma<P>::Frag{};
+#pragma unroll
+      for (int i = 0; i < TS::SN; ++i) b[q][i] = typename Mma<P>::Frag{};
+    }
+  }
+
+  // F32X3: the values of the fragments, and their products on the FP32 MFMA,
+  // element e of both lane halves together.
+  struct Values { float a[NKK][TS::SM][8], b[NKK][TS::SN][8]; };
+  __device__ inline void values(Values& v) const {
+#pragma unroll
+    for (int q = 0; q < NKK; ++q) {
+#pragma unroll
+      for (int j = 0; j < TS::SM; ++j) frag_values(a[q][j], v.a[q][j]);
+#pragma unroll
+      for (int i = 0; i < TS::SN; ++i) frag_values(b[q][i], v.b[q][i]);
+    }
+  }
+  __device__ static inline void mma_f32(typename Mma<P>::Acc (&acc)[TS::SN][TS::SM], const Values& v) {
+#pragma unroll
+    for (int q = 0; q < NKK; ++q)
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+#pragma unroll
+        for (int i = 0; i < TS::SN; ++i)
+#pragma unroll
+          for (int j = 0; j < TS::SM; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(v.b[q][i][e], v.a[q][j][e], acc[i][j], 0, 0, 0);
+  }
 };
 
 // Epilogue through LDS for C layouts whose contiguous runs span both m and
@@ -236,7 +344,7 @@ __device__ inline void store_tile_staged(const GettParams<typename PrecTraits<P>
                                          typename Mma<P>::Acc (&acc)[TileShape<P, BM, BN, BK, WM, WN>::SN]
                                                                     [TileShape<P, BM, BN, BK, WM, WN>::SM],
                                          int m0, int n0, int wm, int wn, int lane, float descale,
-                                         unsigned char* lds_raw, int lds_bytes, bool checker = false) {
+                                         unsigned char* lds_raw, int lds_bytes) {
   using TR = PrecTraits<P>;
   using TG = typename TR::TG;
   using S = TileShape<P, BM, BN, BK, WM, WN>;
@@ -266,7 +374,7 @@ __device__ inline void store_tile_staged(const GettParams<typename PrecTraits<P>
         for (int j = 0; j < S::SM; ++j) {
           TG val = (TG)acc[i][j][r];
           if (P == FP8) val = (TG)((float)val * descale);
-          if (P == BF16X3 && checker && ((lane ^ r) & 1)) val = -val;   // store_tile_from's checker
+          if (P == F32X3) val *= (lane ^ r) & 1 ? -descale : descale;   // as store_tile_from
           L[(n - p0) * LD + wm * S::WTM + j * TR::SUB + m_l] = val;
         }
       }
@@ -450,96 +558,80 @@ __device__ inline void sk_gather(const GettParams<typename PrecTraits<P>::TG>& p
   }
 }
 
-// FP32 through the split-BF16 kernels: whether a pack block under this wave's
-// rows of tile (tm, tn) is held as raw FP32 bits (pack_block).  guardAny is one
-// scalar load per tile; the words are read only when it is set.
-template <int BM, int BN, int WTM, int WTN>
-__device__ inline bool guard_raw(const GettParams<float>& p, int tm, int tn, int wm, int wn, int lane) {
-  if (*p.guardAny == 0u) return false;
-  const int a0 = (tm * BM + wm * WTM) >> 6, a1 = (tm * BM + wm * WTM + WTM - 1) >> 6;
-  const int b0 = (tn * BN + wn * WTN) >> 6, b1 = (tn * BN + wn * WTN + WTN - 1) >> 6;
-  uint32_t raw = 0;
-  for (int i = lane; i < (a1 - a0 + 1) * p.guardK; i += 64) raw |= p.guardA[(size_t)a0 * p.guardK + i];
-  for (int i = lane; i < (b1 - b0 + 1) * p.guardK; i += 64) raw |= p.guardB[(size_t)b0 * p.guardK + i];
-  return __any(raw != 0u);
+// F32X3: whether any pack block of this call holds raw FP32 bits.  The words:
+// [0] and [1] say so for calls in turn, [2] is the turn of the next pack launch,
+// [3] that of the last one (guard_pack_turn, gett_pack.hpp): each pack launch
+// clears the word of the call after it, so nothing has to be cleared between
+// launches and a call's raw blocks cost the calls after it nothing.
+// One load, once per workgroup; `first` (one thread of the GETT kernel) gives the
+// next pack launch the other word.
+__device__ inline bool guard_any(const GettParams<float>& p, bool first) {
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+  const u32x4 w = *reinterpret_cast<const u32x4*>(p.guardAny);
+  const uint32_t turn = w[3] & 1u;
+  if (first) p.guardAny[2] = turn ^ 1u;
+  return (turn ? w[1] : w[0]) != 0u;
 }
 
-// Four consecutive k values of one row of a packed block, as read from its
-// three planes; value(j) is the j-th FP32 value: the raw bits, or the sum of
-// the three parts (exact: the parts do not overlap).
-struct GuardFrag {
-  typedef unsigned short u16x4 __attribute__((ext_vector_type(4)));
-  u16x4 h, m, l;
-  bool raw;
-  template <int F, int BK>
-  __device__ inline void read(const __bf16* blk, int row, int k) {
-    const __bf16* src = blk + chunk_pos<__bf16>(F, row, k >> 3) + (k & 7);
-    h = *reinterpret_cast<const u16x4*>(src);
-    m = *reinterpret_cast<const u16x4*>(src + F * BK);
-    l = *reinterpret_cast<const u16x4*>(src + 2 * F * BK);
+// F32X3: 1 if a pack block under tile (tm, tn) is held as raw FP32 bits
+// (pack_block), 2 if every block of A's or of B's rows is, else 0; the same in
+// every wave, and for every piece of a stream-k tile.
+template <int BM, int BN>
+__device__ inline int tile_raw(const GettParams<float>& p, int tm, int tn) {
+  const int lane = threadIdx.x & 63;
+  uint32_t any = 0, allA = 1, allB = 1;
+  for (int i = lane; i < BM / 64 * p.guardK; i += 64) {
+    const uint32_t w = p.guardA[(size_t)tm * (BM / 64) * p.guardK + i];
+    any |= w;
+    allA &= w;
   }
-  __device__ inline float value(int j) const {
-    const float x0 = __uint_as_float((uint32_t)h[j] << 16), x1 = __uint_as_float((uint32_t)m[j] << 16),
-                x2 = __uint_as_float((uint32_t)l[j] << 16);
-    return raw ? __uint_as_float(((uint32_t)h[j] << 16) | m[j]) : x0 + (x1 + x2);
+  for (int i = lane; i < BN / 64 * p.guardK; i += 64) {
+    const uint32_t w = p.guardB[(size_t)tn * (BN / 64) * p.guardK + i];
+    any |= w;
+    allB &= w;
   }
-};
+  return !__any(any) ? 0 : __all(allA) || __all(allB) ? 2 : 1;
+}
 
-// This wave's part of tile (tm, tn) on the FP32 MFMA, its operands rebuilt
-// from the packed planes: the result of the plain FP32 kernel (same k order,
-// same instruction) for tiles whose operands the split does not hold.  Each
-// wave reads the planes directly (no LDS, no barrier), so it can replace any
-// walk's accumulators right before their epilogue; the next eight k values are
-// in flight during the MFMAs of the current ones.
+// F32X3: adds the k-steps [k0, k0 + KT) of tile (tm, tn) in which this wave's rows
+// have raw blocks, on the FP32 MFMA, to `acc`, which the walk has taken out of the
+// split's scale.  The fragments come from the packed planes directly (no LDS, no
+// barrier); the next such step's are in flight during the MFMAs of one.
 template <int BM, int BN, int BK, int WM, int WN>
-__device__ inline void guard_recompute(const GettParams<float>& p,
-                                       Mma<BF16X3>::Acc (&acc)[TileShape<BF16X3, BM, BN, BK, WM, WN>::SN]
-                                                              [TileShape<BF16X3, BM, BN, BK, WM, WN>::SM],
-                                       int tm, int tn, int wm, int wn, int lane) {
-  using TS = TileShape<BF16X3, BM, BN, BK, WM, WN>;
-  constexpr int BLOCK_A = 3 * BM * BK, BLOCK_B = 3 * BN * BK;
-  const __bf16* Ab = reinterpret_cast<const __bf16*>(p.A) + (size_t)tm * p.kTiles * BLOCK_A;
-  const __bf16* Bb = reinterpret_cast<const __bf16*>(p.B) + (size_t)tn * p.kTiles * BLOCK_B;
-  const int K = p.kTiles * BK;
-  GuardFrag a[TS::SM], b[TS::SN];
-  auto read = [&](int k) {
-    const int kb = k / BK, kin = k - kb * BK + 4 * (lane >> 5);
-#pragma unroll
-    for (int j = 0; j < TS::SM; ++j) {
-      const int row = wm * TS::WTM + j * 32;
-      a[j].raw = p.guardA[(size_t)((tm * BM + row) >> 6) * p.guardK + (k >> 5)] != 0u;
-      a[j].template read<BM, BK>(Ab + (size_t)kb * BLOCK_A, row + (lane & 31), kin);
+__device__ inline void add_raw_steps(const GettParams<float>& p,
+                                     Mma<F32X3>::Acc (&acc)[TileShape<F32X3, BM, BN, BK, WM, WN>::SN]
+                                                           [TileShape<F32X3, BM, BN, BK, WM, WN>::SM],
+                                     int tm, int tn, int wm, int wn, int lane, int k0, int KT) {
+  using FR = PackedFrags<F32X3, BM, BN, BK, WM, WN>;
+  using TS = TileShape<F32X3, BM, BN, BK, WM, WN>;
+  constexpr int BYTES_A = 3 * BM * BK * 2, BYTES_B = 3 * BN * BK * 2;
+  const unsigned char* Ab = reinterpret_cast<const unsigned char*>(p.A) + (size_t)tm * p.kTiles * BYTES_A;
+  const unsigned char* Bb = reinterpret_cast<const unsigned char*>(p.B) + (size_t)tn * p.kTiles * BYTES_B;
+  const int a0 = (tm * BM + wm * TS::WTM) >> 6, a1 = (tm * BM + wm * TS::WTM + TS::WTM - 1) >> 6;
+  const int b0 = (tn * BN + wn * TS::WTN) >> 6, b1 = (tn * BN + wn * TS::WTN + TS::WTN - 1) >> 6;
+  FR f;
+  for (int base = k0; base < k0 + KT; base += 64) {
+    // a lane looks at one k-step
+    uint32_t raw = 0;
+    if (base + lane < k0 + KT) {
+      const int kb = ((base + lane) * BK) >> 5;
+      for (int r = a0; r <= a1; ++r) raw |= p.guardA[(size_t)r * p.guardK + kb];
+      for (int r = b0; r <= b1; ++r) raw |= p.guardB[(size_t)r * p.guardK + kb];
     }
-#pragma unroll
-    for (int i = 0; i < TS::SN; ++i) {
-      const int row = wn * TS::WTN + i * 32;
-      b[i].raw = p.guardB[(size_t)((tn * BN + row) >> 6) * p.guardK + (k >> 5)] != 0u;
-      b[i].template read<BN, BK>(Bb + (size_t)kb * BLOCK_B, row + (lane & 31), kin);
+    uint64_t todo = __ballot(raw != 0u);
+    if (!todo) continue;
+    auto read = [&](uint64_t steps) {
+      const int k = base + __builtin_ctzll(steps);
+      f.read(Ab + (size_t)k * BYTES_A, Bb + (size_t)k * BYTES_B, wm, wn, lane);
+    };
+    read(todo);
+    while (todo) {
+      typename FR::Values v;
+      f.values(v);
+      todo &= todo - 1;
+      if (todo) read(todo);
+      FR::mma_f32(acc, v);
     }
-  };
-#pragma unroll
-  for (int i = 0; i < TS::SN; ++i)
-#pragma unroll
-    for (int j = 0; j < TS::SM; ++j) acc[i][j] = Mma<BF16X3>::Acc{};
-  read(0);
-#pragma unroll 1
-  for (int k = 0; k < K; k += 8) {
-    float va[4][TS::SM], vb[4][TS::SN];
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-#pragma unroll
-      for (int j = 0; j < TS::SM; ++j) va[s][j] = a[j].value(s);
-#pragma unroll
-      for (int i = 0; i < TS::SN; ++i) vb[s][i] = b[i].value(s);
-    }
-    read(k + 8 < K ? k + 8 : k);
-#pragma unroll
-    for (int s = 0; s < 4; ++s)
-#pragma unroll
-      for (int i = 0; i < TS::SN; ++i)
-#pragma unroll
-        for (int j = 0; j < TS::SM; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(vb[s][i], va[s][j], acc[i][j], 0, 0, 0);
   }
 }
 
@@ -547,10 +639,14 @@ __device__ inline void guard_recompute(const GettParams<float>& p,
 // them without a split; part ks of a split-k plan; a stream-k piece with
 // SK), and with PERSIST the tiles of work items v + gridDim.x, ... < nblocks
 // after it.  Every copy into LDS has landed when it returns.
-template <int P, int BM, int BN, int BK, int WM, int WN, int S, bool PERSIST, bool SK = false>
+//
+// RAW (F32X3): tiles with blocks of raw FP32 bits (`raw` as tile_raw() gives it).
+// The walk leaves out the k-steps in which a wave's fragments hold such bits, and
+// add_raw_steps() adds them at its end.
+template <int P, int BM, int BN, int BK, int WM, int WN, int S, bool PERSIST, bool SK = false, bool RAW = false>
 __device__ __forceinline__ void packed_walk(const GettParams<typename PrecTraits<P>::TG>& p, int v, int nblocks,
                                             int tm, int tn, int ks, int k0, int KT, unsigned char* smem_raw,
-                                            const SkPiece& sk = SkPiece{}) {
+                                            const SkPiece& sk = SkPiece{}, int raw = 0) {
   static_assert(!(SK && PERSIST), "a stream-k piece is one tile's k range");
   using SH = PackedShape<P, BM, BN, BK, S>;
   using TS = TileShape<P, BM, BN, BK, WM, WN>;
@@ -604,19 +700,13 @@ __device__ __forceinline__ void packed_walk(const GettParams<typename PrecTraits
     const float b = p.amax[1] > 0.f ? p.amax[1] : 1.f;
     descale = (a / 448.f) * (b / 448.f);
   }
+  if (P == F32X3) descale = kUnscale;
 
   typename MM::Acc acc[TS::SN][TS::SM];
 #pragma unroll
   for (int i = 0; i < TS::SN; ++i)
 #pragma unroll
     for (int j = 0; j < TS::SM; ++j) acc[i][j] = typename MM::Acc{};
-  // A tile that every wave will compute on the FP32 MFMA skips the split.
-  bool all_raw = false;
-  if constexpr (P == BF16X3 && !PERSIST && !SK) {
-    if (p.guardAny && *p.guardAny != 0u)
-      all_raw = __syncthreads_and(guard_raw<BM, BN, TS::WTM, TS::WTN>(p, tm, tn, wm, wn, lane));
-    if (all_raw) KT = 0;
-  }
   // A stream-k piece that finishes its tile adds the earlier pieces' sums.
   // When its segment holds at least a tile's k-steps those were published
   // while the segment's earlier pieces ran: it starts from them, their loads
@@ -624,7 +714,7 @@ __device__ __forceinline__ void packed_walk(const GettParams<typename PrecTraits
   // covers (vmcnt completes in issue order), so their latency hides behind
   // the copies'.  A shorter segment adds them after its own k-steps.
   if constexpr (SK) {
-    if (sk.combine && sk.gather_first) sk_gather<P, BM, BN, BK, WM, WN>(p, acc, sk, w, lane);
+    if (!RAW && sk.combine && sk.gather_first) sk_gather<P, BM, BN, BK, WM, WN>(p, acc, sk, w, lane);
   }
 
   // Fragment double-buffering (the next step's fragments read during this
@@ -643,6 +733,7 @@ __device__ __forceinline__ void packed_walk(const GettParams<typename PrecTraits
   }
 
   int slot = 0;   // stage of the current step
+  bool left_out = false;   // RAW: this wave has left out a k-step of the tile
   int fresh = 0;  // steps left whose awaited copies were issued before the last epilogue
   // one k-step: MFMAs from `cur`; with double-buffering the fragments of the
   // next step go into `nxt`, else `cur` is read from this step's stage first
@@ -666,6 +757,14 @@ __device__ __forceinline__ void packed_walk(const GettParams<typename PrecTraits
       step_sync<(S - 2) * SH::PER_WAVE>();
     }
     const int nslot = (slot + 1 == S) ? 0 : slot + 1;
+    if constexpr (RAW) {
+      // (zeros in place of a branch around the MFMAs, which would cost a second
+      // set of accumulators)
+      if (cur.raw()) {
+        cur.clear();
+        left_out = true;
+      }
+    }
     // One-tile walk: the fragment reads come first in program order (the
     // compiler cannot tell that the copies write another stage, so it keeps
     // them after the reads) and the schedule below spreads both over the
@@ -689,22 +788,7 @@ __device__ __forceinline__ void packed_walk(const GettParams<typename PrecTraits
     // remaining MFMAs; the matrix core is fed from the step's first
     // instruction on.
     if constexpr (DB && !PERSIST) {
-      constexpr int NR = FR::NREAD < FR::NMFMA ? FR::NREAD : FR::NMFMA;
-      constexpr int LEFT = FR::NMFMA - NR;
-      constexpr int NV = SH::PER_WAVE < LEFT ? SH::PER_WAVE : LEFT;
-#pragma unroll
-      for (int i = 0; i < NR; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-      }
-      __builtin_amdgcn_sched_group_barrier(0x100, FR::NREAD - NR, 0);
-#pragma unroll
-      for (int i = 0; i < NV; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-      }
-      __builtin_amdgcn_sched_group_barrier(0x020, SH::PER_WAVE - NV, 0);
-      __builtin_amdgcn_sched_group_barrier(0x008, LEFT - NV, 0);
+      step_schedule<FR::NMFMA, FR::NREAD, SH::PER_WAVE>();
     } else if constexpr (DB) {
       constexpr int NR = FR::NREAD < FR::NMFMA ? FR::NREAD : FR::NMFMA;
       __builtin_amdgcn_sched_group_barrier(0x020, SH::PER_WAVE, 0);
@@ -717,25 +801,37 @@ __device__ __forceinline__ void packed_walk(const GettParams<typename PrecTraits
       __builtin_amdgcn_sched_group_barrier(0x008, FR::NMFMA - NR, 0);
     }
   };
+  // (a tile without a step for the split, not even tried: the persistent walk's
+  // copies depend on every step)
+  const int steps = RAW && !PERSIST && raw == 2 ? 0 : KT;
+  left_out = steps == 0;
   while (true) {
-    for (int k = 0; k + 1 < KT; k += 2) {
+    for (int k = 0; k + 1 < steps; k += 2) {
       step(f0, f1);
       step(f1, f0);
     }
-    if (KT & 1) {
+    if (steps & 1) {
       step(f0, f1);
       if constexpr (DB) f0 = f1;  // the next tile's first fragments
     }
+    if constexpr (RAW) {
+      // (the pieces of a stream-k tile add up without the scale)
+      if (SK || left_out) {
+#pragma unroll
+        for (int i = 0; i < TS::SN; ++i)
+#pragma unroll
+          for (int j = 0; j < TS::SM; ++j) acc[i][j] *= kUnscale;
+      }
+      if (left_out) add_raw_steps<BM, BN, BK, WM, WN>(p, acc, tm, tn, wm, wn, lane, k0, KT);
+      descale = SK || left_out ? 1.f : kUnscale;
+      left_out = false;
+    }
     if constexpr (SK) {
-      if (sk.combine && !sk.gather_first) sk_gather<P, BM, BN, BK, WM, WN>(p, acc, sk, w, lane);
+      if (sk.combine && (RAW || !sk.gather_first)) sk_gather<P, BM, BN, BK, WM, WN>(p, acc, sk, w, lane);
       if (sk.produce) {
         sk_publish<P, BM, BN, BK, WM, WN>(p, acc, sk.slot, w, lane);
         break;
       }
-    }
-    if constexpr (P == BF16X3) {
-      if (p.guardAny && guard_raw<BM, BN, TS::WTM, TS::WTN>(p, tm, tn, wm, wn, lane))
-        guard_recompute<BM, BN, BK, WM, WN>(p, acc, tm, tn, wm, wn, lane);
     }
     if (!PERSIST && ksplit > 1) {
       // raw sums of this k part into the partial-tile buffer, rows n of BM
@@ -759,10 +855,9 @@ __device__ __forceinline__ void packed_walk(const GettParams<typename PrecTraits
       wait_vm_lgkm0<0>();  // the ring is reused for staging: every copy has landed
       __syncthreads();
       store_tile_staged<P, BM, BN, BK, WM, WN>(p, acc, tm * BM, tn * BN, wm, wn, lane, descale, smem_raw,
-                                               SH::LDS_BYTES, P == BF16X3 && p.guardAny);
+                                               SH::LDS_BYTES);
     } else {
-      store_tile<P, BM, BN, BK, WM, WN, PERSIST>(p, acc, tm * BM, tn * BN, wm, wn, lane, descale,
-                                                 P == BF16X3 && p.guardAny);
+      store_tile<P, BM, BN, BK, WM, WN, PERSIST>(p, acc, tm * BM, tn * BN, wm, wn, lane, descale);
     }
     if (!PERSIST) break;
     v += gridDim.x;
@@ -798,6 +893,13 @@ gett_packed_kernel(GettParams<typename PrecTraits<P>::TG> p) {
   // k-steps [k0, k0 + KT) of the tile (all of them without a split)
   const int k0 = (int)((long)ks * p.kTiles / ksplit);
   const int KT = (int)((long)(ks + 1) * p.kTiles / ksplit) - k0;
+  if constexpr (P == F32X3) {
+    const bool any = guard_any(p, v == 0 && threadIdx.x == 0);
+    // (a persistent walk goes from tile to tile without a break: one choice for all)
+    if (const int raw = PERSIST || !any ? any : tile_raw<BM, BN>(p, tm, tn))
+      return packed_walk<P, BM, BN, BK, WM, WN, S, PERSIST, false, true>(p, v, nblocks, tm, tn, ks, k0, KT, smem_raw,
+                                                                         SkPiece{}, raw);
+  }
   packed_walk<P, BM, BN, BK, WM, WN, S, PERSIST>(p, v, nblocks, tm, tn, ks, k0, KT, smem_raw);
 }
 
@@ -829,6 +931,8 @@ gett_packed_sk_kernel(GettParams<typename PrecTraits<P>::TG> p) {
   extern __shared__ __align__(1024) unsigned char smem_raw[];
   const int G = (int)gridDim.x;
   const int g = blockIdx.x;
+  bool any = false;
+  if constexpr (P == F32X3) any = guard_any(p, g == 0 && threadIdx.x == 0);
   const int ntiles = p.tilesM * p.tilesN;
   const int rounds = ntiles / G;
   const int dp = rounds > kSkTailRounds ? (rounds - kSkTailRounds) * G : 0;   // tiles walked whole
@@ -873,6 +977,12 @@ gett_packed_sk_kernel(GettParams<typename PrecTraits<P>::TG> p) {
     // the previous piece's LDS reads (fragments, staged C) are done before
     // this piece's copies overwrite the ring
     if (i) __syncthreads();
+    if constexpr (P == F32X3) {
+      if (const int raw = any ? tile_raw<BM, BN>(p, tm, tn) : 0) {
+        packed_walk<P, BM, BN, BK, WM, WN, S, false, true, true>(p, 0, ntiles, tm, tn, 0, k0, nk, smem_raw, sk, raw);
+        continue;
+      }
+    }
     packed_walk<P, BM, BN, BK, WM, WN, S, false, true>(p, 0, ntiles, tm, tn, 0, k0, nk, smem_raw, sk);
   }
 }

@@ -9,13 +9,3 @@ extern "C" int tccg_gett_packed_bf16x3(const float* A, const float* B, float* C,
                                     void* stream) {
   return tccg_lib::run_gett_packed<tccg::BF16X3>(A, B, C, alpha, beta, plan, workspace, workspace_bytes, stream);
 }
-
-// FP32 results through the split: pack blocks whose values the three parts do
-// not hold exactly keep their FP32 bits, and the tiles that read them run on
-// the FP32 MFMA (gett_pack.hpp split_holds(), gett_packed.hpp guard_recompute()).
-extern "C" int tccg_gett_f32_split(const float* A, const float* B, float* C, float alpha, float beta,
-                                   const tccg_gett_plan* plan, void* workspace, size_t workspace_bytes,
-                                   int prepacked, void* stream) {
-  return tccg_lib::run_gett_packed<tccg::BF16X3>(A, B, C, alpha, beta, plan, workspace, workspace_bytes, stream,
-                                                 !prepacked, true);
-}

@@ -130,7 +130,7 @@ class GettGroup:
         return len(self._probs) - 1
 
     def _header(self) -> int:
-        """Bytes before the first operand: the word that any raw block sets."""
+        """Bytes before the first operand: the words that say whether any raw block is there."""
         return 256 if self.guard else 0
 
     def plane_bytes(self, op) -> int:
@@ -249,7 +249,7 @@ class GettGroup:
         elif workspace.dtype != torch.uint8 or workspace.numel() < need or workspace.device != dev:
             raise ValueError("group workspace must be a uint8 tensor of >= %d bytes on %s" % (need, dev))
         if self.guard:
-            workspace[:4].copy_(torch.zeros(4, dtype=torch.uint8))
+            workspace[:16].copy_(torch.zeros(16, dtype=torch.uint8))
         up = lambda arr: torch.from_numpy(np.frombuffer(bytes(arr), dtype=np.uint8).copy()).to(dev)
         self._bound = dict(tables=tables, ops=up(ops), nops=len(self._ops), jobs=torch.from_numpy(jobs).to(dev),
                            njobs=int(jobs.shape[0]), probs=up(probs), nprobs=len(self._probs),

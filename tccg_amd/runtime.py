@@ -262,11 +262,11 @@ class DevicePlan:
             else:
                 self.workspace = torch.empty(nbytes, dtype=torch.uint8, device=dev)
             if plan.guard:
-                # the word that any pack block with raw values sets: while it is
-                # clear, no tile has to look at its guard words (a copy from the
-                # host: done on return, whatever stream the first call runs on)
+                # the words that say whether any pack block holds raw values
+                # (a copy from the host: done on return, whatever stream the
+                # first call runs on)
                 off = lib.tccg_f32_split_clear_offset(ctypes.byref(c))
-                self.workspace[off:off + 4].copy_(torch.zeros(4, dtype=torch.uint8))
+                self.workspace[off:off + 16].copy_(torch.zeros(16, dtype=torch.uint8))
 
         # what every call needs again: the expected tensors (.tccg order) and the
         # arguments that do not change

@@ -12,32 +12,39 @@ from tccg_amd.plan import (BF16X3, F32, F64, PACKED_TAIL_BYTES, SPLIT_MIN_K, bui
                            default_plan, split_plans)
 
 
-def holds(x: np.ndarray) -> np.ndarray:
-    """split_holds() of gett_pack.hpp."""
-    u = np.ascontiguousarray(x, np.float32).view(np.uint32)
-    return ((u << np.uint32(1)) == 0) | (((u >> np.uint32(23)) & np.uint32(0xff)) - np.uint32(27) <= np.uint32(150))
+SCALE = 23   # kSplitScale of gett_core.hpp: the parts are those of x 2^23
 
 
-@pytest.mark.parametrize("e", [-100, -99, -1, 0, 1, 49, 50])
+def limit(Kp: int) -> int:
+    """h of split_limit() in gett_pack.hpp: |x| < 2^h is held."""
+    return (81 - (Kp - 1).bit_length()) // 2
+
+
+@pytest.mark.parametrize("e", [-149, -148, -140, -127, -126, -125, -100, -1, 0, 1, 33, 37])
 def test_parts_hold_every_accepted_value(e):
-    """Every mantissa pattern class at the edges of the accepted exponents: the
-    three parts add up to the value exactly, in FP32 from the smallest up, and
-    each is zero or a normal BF16 number."""
+    """Every mantissa pattern class at the edges of the accepted exponents,
+    subnormals among them: the three parts add up to the scaled value exactly, in
+    FP32 from the smallest up, and each is zero or a normal BF16 number."""
     rng = np.random.default_rng(e + 200)
     man = np.concatenate([np.arange(64), (1 << 23) - 1 - np.arange(64), rng.integers(0, 1 << 23, 20000),
                           (rng.integers(0, 128, 500) << 16) | 0x8000, (rng.integers(0, 1 << 15, 500) << 8) | 0x80])
     x = np.concatenate([s * np.ldexp(1.0 + man / 2.0 ** 23, e) for s in (1, -1)]).astype(np.float32)
-    assert holds(x).all()
-    p0, p1, p2 = (p.astype(np.float32) for p in split_bf16_parts(x))
-    assert np.array_equal(p0 + (p1 + p2), x)
+    xs = x * np.float32(2.0 ** SCALE)
+    assert np.array_equal(xs.astype(np.float64), x.astype(np.float64) * 2.0 ** SCALE)
+    p0, p1, p2 = (p.astype(np.float32) for p in split_bf16_parts(xs))
+    assert np.array_equal(p0 + (p1 + p2), xs)
     for p in (p0, p1, p2):
-        assert np.all((p == 0) | ((np.abs(p) >= 2.0 ** -126) & (np.abs(p) <= 2.0 ** 51)))
+        assert np.all((p == 0) | (np.abs(p) >= 2.0 ** -126))
 
 
-def test_values_that_are_not_held():
-    x = np.array([np.inf, -np.inf, np.nan, 3e38, 2.0 ** 51, 2.0 ** -101, 1e-39, -1e-45], np.float32)
-    assert not holds(x).any()
-    assert holds(np.array([0.0, -0.0, 2.0 ** -100, np.nextafter(np.float32(2.0 ** 51), np.float32(0))], np.float32)).all()
+@pytest.mark.parametrize("Kp", [32, 64, 96, 2304, 4096, 4128, 1 << 20])
+def test_held_values_cannot_overflow(Kp):
+    """Kp products of the largest first parts (2^(h + 23) each) stay under 2^127,
+    and the limit is the largest that a sum of Kp products allows in this form."""
+    h = limit(Kp)
+    assert Kp * 2.0 ** (2 * (h + SCALE)) <= 2.0 ** 127
+    assert 2.0 ** (Kp - 1).bit_length() * 2.0 ** (2 * (h + 1 + SCALE)) > 2.0 ** 127
+    assert h >= 27
 
 
 def _matmul(m, n, k):

@@ -36,6 +36,7 @@ def _specials(A, B):
     A[5, 7], A[-2, -1], A[130, 33], A[70, 3] = np.inf, np.nan, 3.0e38, 1e-39
     A[40, :] *= 2.0 ** -120
     B[1, 20], B[-1, 100], B[4, 65], B[:, 3] = -np.inf, 1e-35, 2.0 ** 60, B[:, 3] * np.float32(2.0 ** -110)
+    A[200, 40:], B[70:, 200] = 2.0 ** 40, -2.0 ** 41
     return A, B
 
 
@@ -60,6 +61,91 @@ def test_special_values_give_the_fp32_result(tile, walk):
         ok = np.isfinite(out)
         bound = (k + 8) * 2.0 ** -23 * mag[ok] + 2.0 ** -125
         assert np.all(np.abs(out[ok] - ref[ok]) <= bound)
+
+
+def _words(dp):
+    """(whether the last call packed a raw block, its pack blocks' words) of a
+    guarded DevicePlan."""
+    import ctypes
+    import torch
+    from tccg_amd.runtime import load_library
+    off = load_library().tccg_f32_split_clear_offset(ctypes.byref(dp.cplan))
+    n = (dp.plan.Mp // 64 + dp.plan.Np // 64) * (dp.plan.Kp // 32)
+    head = dp.workspace[off:off + 16].view(torch.int32).cpu().numpy()
+    return int(head[head[3] & 1]), dp.workspace[off + 256:off + 256 + 4 * n].view(torch.int32).cpu().numpy()
+
+
+def test_values_of_every_size_are_held_and_raw_blocks_cost_one_call():
+    """Operands over the whole range below the limit, subnormals included, have no
+    raw block; a larger value, an infinity or a NaN makes its own pack block raw,
+    and the next call's tiles look at no words for it."""
+    import torch
+    from tccg_amd.runtime import DevicePlan
+    c = _matmul(200, 150, 130)
+    rng = np.random.default_rng(7)
+    wide = lambda s: np.ldexp(rng.uniform(-2, 2, s), rng.integers(-149, 34, s)).astype(np.float32)
+    A, B = wide(c.shapes()[0]), wide(c.shapes()[1])
+    dev = lambda x: torch.from_numpy(np.ascontiguousarray(x)).cuda()
+    dp = DevicePlan(_split(c, 0))
+    C = torch.zeros(c.shapes()[2], device="cuda")
+    dp.run(dev(A), dev(B), C)
+    torch.cuda.synchronize()
+    any_, words = _words(dp)
+    assert any_ == 0 and not words.any()
+    for value in (np.inf, np.nan, 2.0 ** 36):
+        As = A.copy()
+        As[70, 40] = value
+        dp.run(dev(As), dev(B), C)
+        torch.cuda.synchronize()
+        any_, words = _words(dp)
+        nk = dp.plan.Kp // 32
+        assert any_ == 1 and words.sum() == 1 and words[(70 // 64) * nk + 40 // 32] == 1   # A's m is the free set
+        dp.run(dev(A), dev(B), C)
+        torch.cuda.synchronize()
+        any_, words = _words(dp)
+        assert any_ == 0 and not words.any()
+
+
+@pytest.mark.parametrize("walk", range(3))
+@pytest.mark.parametrize("where", ["few", "half", "A", "both"])
+def test_raw_steps_over_long_k(walk, where):
+    """More k-steps than a wave looks at together (64), raw blocks in a few, in
+    half and in all of them: against FP64 with the bound of k rounded additions."""
+    m, n, k = 200, 150, (2100 if walk != 1 else 250)
+    c = _matmul(m, n, k)
+    A, B, _ = inputs(c, 31)
+    rng = np.random.default_rng(5)
+    if where == "few":
+        A[7, 5], A[150, k - 1], B[k // 2, 3] = 2.0 ** 50, -2.0 ** 45, 2.0 ** 47
+    elif where == "half":
+        A[:, rng.permutation(-(-k // 32))[:k // 64] * 32] *= np.float32(2.0 ** 45)
+    else:
+        A *= np.float32(2.0 ** 45)
+        if where == "both":
+            B *= np.float32(2.0 ** 45)
+    for tile in (0, 4, 6):
+        plan = _split(c, tile, **WALKS[walk])
+        print(plan.describe(), flush=True)
+        out = run_gpu(c, A, B, np.zeros(c.shapes()[2], np.float32), prec=F32, plan=plan)
+        ref, mag = _exact(A, B, np.zeros(c.shapes()[2], np.float32), 1.0, 0.0)
+        assert np.all(np.abs(out - ref) <= (k + 8) * 2.0 ** -23 * mag)
+
+
+@pytest.mark.parametrize("ea, eb", [(-62, -62), (-63, -63), (-99, -20), (-120, 0), (-140, 14), (-65, -65)])
+def test_products_at_the_bottom_of_the_range(ea, eb):
+    """Held operands whose products lie around FP32's smallest normal number: the
+    low products of the parts must not be lost.  The error is at most the FP32
+    kernel's, but for one rounding to a subnormal result (2^-150)."""
+    c = _matmul(128, 128, 64)
+    rng = np.random.default_rng(1)
+    mk = lambda s, e: (np.ldexp(rng.uniform(1, 2, s), e) * rng.choice([-1, 1], s)).astype(np.float32)
+    A, B = mk(c.shapes()[0], ea), mk(c.shapes()[1], eb)
+    C = np.zeros(c.shapes()[2], np.float32)
+    ref, _ = _exact(A, B, C, 1.0, 0.0)
+    err = lambda plan: np.sqrt(np.mean((run_gpu(c, A, B, C, prec=F32, plan=plan) - ref) ** 2))
+    split, fp32 = err(_split(c, 0)), err(build_packed_plan(c.problem, F32, 2))
+    print("2^%d 2^%d: split %.3e, FP32 MFMA %.3e (in 2^-149)" % (ea, eb, split * 2.0 ** 149, fp32 * 2.0 ** 149), flush=True)
+    assert split <= fp32 + 2.0 ** -150
 
 
 @pytest.mark.parametrize("k", [32, 100, 2304])
