@@ -539,11 +539,12 @@ __device__ inline void store_tile_from(const GettParams<typename PrecTraits<P>::
   using S = TileShape<P, BM, BN, BK, WM, WN>;
   using MM = Mma<P>;
   // F32X3: the accumulators hold (-1)^(m + n) C over `descale` (pack_block); m's
-  // parity is the lane's, n's that of the accumulator register.
+  // parity is the lane's, n's that of the accumulator register.  The sum with
+  // zero leaves no negative zero where C is zero.
   const TG alpha = p.alpha, beta = p.beta;
   const float sign[2] = {lane & 1 ? -descale : descale, lane & 1 ? descale : -descale};
   auto value = [&](const typename MM::Acc& a, int r) {
-    if constexpr (P == F32X3) return sign[r & 1] * a[r];
+    if constexpr (P == F32X3) return __builtin_fmaf(sign[r & 1], a[r], 0.f);
     else if constexpr (P == FP8) return (TG)((float)a[r] * descale);
     else return (TG)a[r];
   };

@@ -374,7 +374,7 @@ __device__ inline void store_tile_staged(const GettParams<typename PrecTraits<P>
         for (int j = 0; j < S::SM; ++j) {
           TG val = (TG)acc[i][j][r];
           if (P == FP8) val = (TG)((float)val * descale);
-          if (P == F32X3) val *= (lane ^ r) & 1 ? -descale : descale;   // as store_tile_from
+          if (P == F32X3) val = __builtin_fmaf((lane ^ r) & 1 ? -descale : descale, val, 0.f);   // store_tile_from
           L[(n - p0) * LD + wm * S::WTM + j * TR::SUB + m_l] = val;
         }
       }

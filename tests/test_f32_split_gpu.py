@@ -106,6 +106,49 @@ def test_values_of_every_size_are_held_and_raw_blocks_cost_one_call():
         assert any_ == 0 and not words.any()
 
 
+def _zero_inputs(c, seed, raw):
+    """Whole numbers; C is zero where a row of A or a column of B is, and where
+    the two halves of k cancel."""
+    rng = np.random.default_rng(seed)
+    sa, sb, _ = c.shapes()
+    A, B = (rng.integers(-9, 10, s).astype(np.float32) for s in (sa, sb))
+    k = sa[1]                                            # A (c, k, a), B (b, d, k)
+    A[:, k // 2:, ::3], B[:, ::2, k // 2:] = A[:, :k // 2, ::3], -B[:, ::2, :k // 2]
+    A[5], B[7] = 0, 0
+    if raw:
+        A[20, 3, 1] = 2.0 ** 60
+    return A, B
+
+
+@pytest.mark.parametrize("raw", [False, True])
+@pytest.mark.parametrize("alpha", [1.5, -1.5])
+def test_zeros_have_the_sign_of_the_fp32_kernel(alpha, raw):
+    """The epilogues undo the sign of the packed rows: zeros come out as +0 (times
+    alpha) all the same, from the direct and the run epilogue, the persistent and
+    the stream-k walk, and in a group."""
+    import torch
+    from tccg_amd.batch import GettBatch
+    c = Contraction.from_labels(list("abcd"), list("akc"), list("kdb"), dict(a=24, b=24, c=24, d=24, k=64))
+    A, B = _zero_inputs(c, 2, raw)
+    C = np.zeros(c.shapes()[2], np.float32)
+    fp32 = run_gpu(c, A, B, C, prec=F32, alpha=alpha, plan=build_packed_plan(c.problem, F32, 2))
+    assert np.count_nonzero(fp32 == 0) > fp32.size // 8
+    runs = 0
+    for tile, kw in [(0, {}), (6, {}), (0, WALKS[1]), (6, WALKS[1]), (4, WALKS[2])]:
+        plan = _split(c, tile, **kw)
+        runs += plan.crun[0] > 0 and not plan.grid
+        out = run_gpu(c, A, B, C, prec=F32, alpha=alpha, plan=plan)
+        assert np.array_equal(out, fp32), plan.describe()   # whole numbers: exact
+        assert np.array_equal(np.signbit(out), np.signbit(fp32)), plan.describe()
+    assert runs
+    dev = lambda x: torch.from_numpy(np.ascontiguousarray(x)).cuda()
+    Cs = [torch.zeros(c.shapes()[2], device="cuda")]
+    b = GettBatch([c], alphas=[alpha], betas=[0.0], group_tile=PACKED_TILES[F32].index((128, 128, 16)))
+    b.bind([dev(A)], [dev(B)], Cs).launch()
+    torch.cuda.synchronize()
+    assert np.array_equal(np.signbit(Cs[0].cpu().numpy()), np.signbit(fp32))
+
+
 @pytest.mark.parametrize("walk", range(3))
 @pytest.mark.parametrize("where", ["few", "half", "A", "both"])
 def test_raw_steps_over_long_k(walk, where):
