@@ -20,7 +20,7 @@ from typing import Dict, List, Optional, Sequence
 import numpy as np
 
 from .contraction import Contraction
-from .plan import BF16X3, F32, PACKED_TILES, TILES, build_packed_plan, build_plan, split_fits
+from .plan import (BF16X3, F32, PACKED_TILES, SPLIT_RESIDENT, TILES, build_packed_plan, build_plan, split_fits)
 
 # batch shape id -> tile id of TILES[F32] with the same (BM, BN, BK)
 BATCH_SHAPES = {0: TILES[F32].index((64, 64, 32)), 1: TILES[F32].index((128, 128, 32))}
@@ -43,24 +43,32 @@ def pattern_key(c: Contraction) -> str:
 LARGE_TILE = PACKED_TILES[F32].index((128, 128, 16))
 
 
-# Shortest k range of a batch that runs on the BF16 MFMAs: from k = 4 on the
+# Shortest k range of a batch that runs on the BF16 MFMAs: from k = 2 on the
 # split's error is no larger than the FP32 MFMA's (plan.SPLIT_MIN_K); grouped
 # problems pay no pack launch of their own, so the rule is accuracy's alone.
 GROUP_SPLIT_MIN_K = 4
 
 
+def group_split_tile(tile: int) -> Optional[int]:
+    """The split-BF16 tile that a grouped launch with FP32 packed tile `tile`
+    runs on where it may: that of the same shape, or 192x128 for shapes whose
+    accumulators do not stay in registers there; None without one."""
+    BM, BN, BK = PACKED_TILES[F32][tile]
+    same = [t for t in SPLIT_RESIDENT if PACKED_TILES[BF16X3][t][:2] == (BM, BN)]
+    if same:
+        return min(same, key=lambda t: PACKED_TILES[BF16X3][t][2] != BK)
+    return PACKED_TILES[BF16X3].index((192, 128, 16)) if (BM, BN, 16) in PACKED_TILES[BF16X3] else None
+
+
 def group_plans(contractions: Sequence[Contraction], tile: int):
     """The packed plans of a grouped launch with FP32 packed tile `tile`: the
-    guarded split-BF16 plans of the same tile where one exists and every
-    contraction may take it (they beat the FP32 MFMA at every batch measured:
-    40 problems of the batch patterns 3.32 -> 2.21 ms, 512 40.8 -> 28.2 ms), else the FP32 plans."""
-    BM, BN, _ = PACKED_TILES[F32][tile]
-    same = [t for t, s in enumerate(PACKED_TILES[BF16X3]) if s[:2] == (BM, BN)]
-    if same and all(c.problem.K >= GROUP_SPLIT_MIN_K for c in contractions):
-        plans = [build_packed_plan(c.problem, BF16X3, same[0]) for c in contractions]
+    guarded split-BF16 plans of group_split_tile() where every contraction may
+    take them (they beat the FP32 MFMA at every batch measured: 40 problems of the
+    batch patterns 3.32 -> 2.14 ms), else the FP32 plans."""
+    split = group_split_tile(tile)
+    if split is not None and all(c.problem.K >= GROUP_SPLIT_MIN_K for c in contractions):
+        plans = [build_packed_plan(c.problem, BF16X3, split, guard=True) for c in contractions]
         if all(split_fits(p) for p in plans):
-            for p in plans:
-                p.guard = True
             return plans
     return [build_packed_plan(c.problem, F32, tile) for c in contractions]
 

@@ -386,9 +386,36 @@ template <> struct Mma<F64> {
 };
 
 struct Bf16x3Frag { bf16x8 p[3]; };
+
+// Two sums per element of C in the split precisions.  `hi` takes a0 b0, whose
+// products are exact in FP32, so that 16 k values cost one rounding at full
+// size; `lo` takes the five smaller products, 2^-8 of it and their roundings
+// with them.  In one sum each of the six MFMAs rounds at its full size: where few
+// products make up an element that was up to 2.0 times the FP32 MFMA's error (8
+// to 32 nonzero values in rows of 512: 1.06e-7 against 5.3e-8, with two sums
+// 2.8e-8; dense rows of 4096, N(0, 1): 1.0e-6 against 1.14e-6, 4.0e-7).
+struct PairAcc {
+  f32x16 hi, lo;
+  __device__ inline float operator[](int r) const { return hi[r] + lo[r]; }
+  __device__ inline void add(int r, float v) { hi[r] += v; }
+  __device__ inline void fold() {
+    hi += lo;
+    lo = f32x16{};
+  }
+  __device__ inline void scale(float s) {
+    hi = (hi + lo) * s;
+    lo = f32x16{};
+  }
+};
+
+// FP32 through the split (F32X3): the parts are those of the operand values
+// times kSplitScale (gett_pack.hpp split_limit()), the sums hold C times its
+// square.
+constexpr float kSplitScale = 0x1p23f, kUnscale = 0x1p-46f;
+
 template <> struct Mma<BF16X3> {
   using Frag = Bf16x3Frag;
-  using Acc = f32x16;
+  using Acc = PairAcc;
   static constexpr int NACC = 16;
   __device__ static inline Frag read(const __bf16* lds, int plane_stride, int row0, int kk, int LDK, int lane) {
     Frag f;
@@ -397,13 +424,14 @@ template <> struct Mma<BF16X3> {
     for (int q = 0; q < 3; ++q) f.p[q] = *reinterpret_cast<const bf16x8*>(lds + q * plane_stride + idx);
     return f;
   }
-  // product q of (b part, a part): (0,2) (1,1) (2,0) (0,1) (1,0) (0,0),
-  // smallest terms first
+  // product q of (b part, a part): (0,2) (1,1) (2,0) (0,1) (1,0), smallest terms
+  // first, and (0,0)
   static constexpr int PARTS = 6;
   __device__ static inline void mma_part(Acc& acc, const Frag& b, const Frag& a, int q) {
     constexpr int bi[6] = {0, 1, 2, 0, 1, 0};
     constexpr int ai[6] = {2, 1, 0, 1, 0, 0};
-    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b.p[bi[q]], a.p[ai[q]], acc, 0, 0, 0);
+    f32x16& sum = q < PARTS - 1 ? acc.lo : acc.hi;
+    sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b.p[bi[q]], a.p[ai[q]], sum, 0, 0, 0);
   }
   __device__ static inline void mma(Acc& acc, const Frag& b, const Frag& a) {
 #pragma unroll
@@ -415,9 +443,6 @@ template <> struct Mma<BF16X3> {
   }
 };
 
-// FP32 through the split.  The parts are those of the operand values times
-// kSplitScale (gett_pack.hpp split_limit()); the sums hold C times its square.
-constexpr float kSplitScale = 0x1p23f, kUnscale = 0x1p-46f;
 template <> struct Mma<F32X3> : Mma<BF16X3> {};
 
 template <> struct Mma<BF16> {

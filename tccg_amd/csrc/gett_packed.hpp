@@ -92,9 +92,9 @@ struct PackedShape {
   static constexpr int STAGE_BYTES = BYTES_A + BYTES_B;
   static constexpr int LDS_BYTES = S * STAGE_BYTES;
   static constexpr int NA = BYTES_A / 1024, NB = BYTES_B / 1024;  // kilobyte copies per k-step
-  static constexpr int PER_WAVE = (NA + NB) / 4;
+  // (where the four waves cannot share them evenly, the last ones copy the last kilobyte again)
+  static constexpr int PER_WAVE = (NA + NB + 3) / 4;
   static_assert(BYTES_A % 1024 == 0 && BYTES_B % 1024 == 0, "k-step blocks are whole kilobytes");
-  static_assert((NA + NB) % 4 == 0, "copies divide evenly over the four waves");
   static_assert((BK * (int)sizeof(TL)) % 32 == 0, "rows of whole 32-byte sub-rows");
   // copies run S steps ahead with fragment double-buffering (S - 1 without, FP8)
   static_assert(S >= (P == FP8 ? 2 : 3) && S * PER_WAVE < 64, "ring depth");
@@ -163,7 +163,7 @@ __device__ inline void packed_copy(const unsigned char* gA, const unsigned char*
   using SH = PackedShape<P, BM, BN, BK, S>;
 #pragma unroll
   for (int j = 0; j < SH::PER_WAVE; ++j) {
-    const int i = w + 4 * j;
+    const int i = min(w + 4 * j, SH::NA + SH::NB - 1);
     const bool isA = i < SH::NA;
     const unsigned char* src = (isA ? gA + i * 1024 : gB + (i - SH::NA) * 1024) + lane * 16;
     unsigned char* dst = stage + (isA ? i * 1024 : SH::BYTES_A + (i - SH::NA) * 1024);
@@ -194,14 +194,14 @@ struct PackedCopier {
     tB = gB;
 #pragma unroll
     for (int j = 0; j < SH::PER_WAVE; ++j) {
-      const int i = w + 4 * j;
+      const int i = min(w + 4 * j, SH::NA + SH::NB - 1);
       voff[j] = (uint32_t)((is_a(w, j) ? i : i - SH::NA) * 1024 + lane * 16);
     }
   }
   __device__ inline void issue(unsigned char* stage, int w) const {
 #pragma unroll
     for (int j = 0; j < SH::PER_WAVE; ++j)
-      __builtin_amdgcn_global_load_lds((is_a(w, j) ? tA : tB) + voff[j], stage + (w + 4 * j) * 1024, 16, 0, 0);
+      __builtin_amdgcn_global_load_lds((is_a(w, j) ? tA : tB) + voff[j], stage + min(w + 4 * j, SH::NA + SH::NB - 1) * 1024, 16, 0, 0);
   }
   __device__ inline void advance() {
     tA += SH::BYTES_A;
@@ -330,7 +330,7 @@ struct PackedFrags {
         for (int i = 0; i < TS::SN; ++i)
 #pragma unroll
           for (int j = 0; j < TS::SM; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(v.b[q][i][e], v.a[q][j][e], acc[i][j], 0, 0, 0);
+            acc[i][j].hi = __builtin_amdgcn_mfma_f32_32x32x2f32(v.b[q][i][e], v.a[q][j][e], acc[i][j].hi, 0, 0, 0);
   }
 };
 
@@ -477,18 +477,44 @@ __device__ inline void sk_add_partial(const GettParams<typename PrecTraits<P>::T
   using TS = TileShape<P, BM, BN, BK, WM, WN>;
   using SL = SkSlot<P, BM, BN, BK, WM, WN>;
   const __amdgpu_buffer_rsrc_t r = SL::rsrc(p, slot);
+  constexpr int QA = SL::NACC / SL::VEC;   // vectors per accumulator
+  if constexpr (PrecTraits<P>::PLANES == 3) {
+    // Left to itself the compiler loads a vector, waits and adds it, one after
+    // the other, beside the pairs' registers (204 x 1560, k = 2205, 128x128
+    // tiles, ten pieces a tile: 82 us, 48 with one sum): up to 16 go out together.
+    constexpr int GRP = SL::NV < 16 ? SL::NV : 16;
 #pragma unroll
-  for (int i = 0; i < TS::SN; ++i)
+    for (int g = 0; g < SL::NV; g += GRP) {
+      typename SL::V v[GRP];
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int j = 0; j < TS::SM; ++j)
+      for (int e = 0; e < GRP; ++e)
+        if (g + e < SL::NV)
+          v[e].bits = __builtin_amdgcn_raw_buffer_load_b128(r, ((w * SL::NV + g + e) * 64 + lane) * 16, 0, CPOL);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int q = 0; q < SL::NACC / SL::VEC; ++q) {
-        const int vq = (i * TS::SM + j) * (SL::NACC / SL::VEC) + q;
-        typename SL::V v;
-        v.bits = __builtin_amdgcn_raw_buffer_load_b128(r, ((w * SL::NV + vq) * 64 + lane) * 16, 0, CPOL);
+      for (int e = 0; e < GRP; ++e)
+        if (g + e < SL::NV) {
+          const int vq = g + e, i = vq / QA / TS::SM, j = vq / QA % TS::SM;
 #pragma unroll
-        for (int e = 0; e < SL::VEC; ++e) acc[i][j][q * SL::VEC + e] += v.e[e];
-      }
+          for (int x = 0; x < SL::VEC; ++x) acc[i][j].add(vq % QA * SL::VEC + x, v[e].e[x]);
+        }
+    }
+    return;
+  } else {
+#pragma unroll
+    for (int i = 0; i < TS::SN; ++i)
+#pragma unroll
+      for (int j = 0; j < TS::SM; ++j)
+#pragma unroll
+        for (int q = 0; q < QA; ++q) {
+          const int vq = (i * TS::SM + j) * QA + q;
+          typename SL::V v;
+          v.bits = __builtin_amdgcn_raw_buffer_load_b128(r, ((w * SL::NV + vq) * 64 + lane) * 16, 0, CPOL);
+#pragma unroll
+          for (int e = 0; e < SL::VEC; ++e) acc[i][j][q * SL::VEC + e] += v.e[e];
+        }
+  }
 }
 
 template <int P, int BM, int BN, int BK, int WM, int WN>
@@ -650,6 +676,7 @@ __device__ __forceinline__ void packed_walk(const GettParams<typename PrecTraits
   static_assert(!(SK && PERSIST), "a stream-k piece is one tile's k range");
   using SH = PackedShape<P, BM, BN, BK, S>;
   using TS = TileShape<P, BM, BN, BK, WM, WN>;
+  using TR = PrecTraits<P>;
   using MM = Mma<P>;
   using FR = PackedFrags<P, BM, BN, BK, WM, WN>;
   const int ntiles = p.tilesM * p.tilesN;
@@ -820,11 +847,19 @@ __device__ __forceinline__ void packed_walk(const GettParams<typename PrecTraits
 #pragma unroll
         for (int i = 0; i < TS::SN; ++i)
 #pragma unroll
-          for (int j = 0; j < TS::SM; ++j) acc[i][j] *= kUnscale;
+          for (int j = 0; j < TS::SM; ++j) acc[i][j].scale(kUnscale);
       }
       if (left_out) add_raw_steps<BM, BN, BK, WM, WN>(p, acc, tm, tn, wm, wn, lane, k0, KT);
       descale = SK || left_out ? 1.f : kUnscale;
       left_out = false;
+    }
+    if constexpr (SK && TR::PLANES == 3 && !RAW) {
+      // one sum before the pieces' are added: both together leave too few
+      // registers for the partial's loads
+#pragma unroll
+      for (int i = 0; i < TS::SN; ++i)
+#pragma unroll
+        for (int j = 0; j < TS::SM; ++j) acc[i][j].fold();
     }
     if constexpr (SK) {
       if (sk.combine && (RAW || !sk.gather_first)) sk_gather<P, BM, BN, BK, WM, WN>(p, acc, sk, w, lane);

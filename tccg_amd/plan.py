@@ -56,10 +56,14 @@ PACKED_TILES: Dict[int, List[Tuple[int, int, int]]] = {
           (192, 64, 16), (192, 192, 32)],
     F64: [(128, 128, 16), (64, 64, 16)],
     BF16X3: [(128, 128, 16), (128, 128, 32), (256, 128, 16), (128, 256, 16), (64, 64, 32), (192, 192, 16),
-             (192, 64, 16)],
+             (192, 64, 16), (192, 128, 16), (128, 192, 16)],
     FP8: [(128, 128, 128), (256, 128, 128), (64, 64, 128), (192, 192, 128), (192, 64, 128)],
     BF16: [(128, 128, 32), (256, 128, 32), (128, 256, 32), (64, 64, 32), (192, 192, 32), (192, 64, 32)],
 }
+# Split-BF16 packed tiles that plans are chosen from: those whose pairs of
+# accumulators stay in registers.  256x128, 128x256 and 192x192 keep some in
+# memory (5184 x 5184, k = 2304: 668, 659 and 1681 us; 192x128 579, 128x192 575).
+SPLIT_RESIDENT = (0, 1, 4, 6, 8, 7)
 # Tiles of the vector micro-kernel (walk 3) for short k ranges, FP32 and FP64:
 # BM m positions x BN n positions, BK = the whole padded k range
 # (csrc/gett_launch.hpp kF32VecTiles / kF64VecTiles).
@@ -506,7 +510,7 @@ def _store_run(offCm: np.ndarray, offCn: np.ndarray, BM: int) -> int:
 
 def build_packed_plan(pb: GettProblem, prec: int, tile: int, groupM: int = 8,
                       persistent: bool = False, store_waves: bool = False, ksplit: int = 1,
-                      stream_k: int = 0) -> GettPlan:
+                      stream_k: int = 0, guard: bool = False) -> GettPlan:
     """Plan of the packed path: the reference's pack-then-macro-kernel GETT
     (tccg/gett.py:346-391, tccg/gett.py:1092-1098) with each operand packed
     once.  Plain linearisations (the pack kernel reads every element once, so
@@ -516,7 +520,10 @@ def build_packed_plan(pb: GettProblem, prec: int, tile: int, groupM: int = 8,
     stride-one index is contracted, else FREE1.  stream_k > 0: the stream-k
     walk over stream_k workgroups per CU (every k-step of every tile spread
     evenly over the grid; the reference balances its loops over threads by
-    cost, tccg/gett.py:755-959)."""
+    cost, tccg/gett.py:755-959).  guard (split-BF16): an FP32 contraction
+    through the split."""
+    if guard and (prec != BF16X3 or store_waves or ksplit > 1):
+        raise ValueError("FP32 through the split runs on the split-BF16 kernels, walk 0 or 5 without ksplit")
     BM, BN, BK = PACKED_TILES[prec][tile]
     m_l, n_l, k_l = _orders(pb)
     lin_m = Linearization.plain(m_l, _ext(pb, m_l))
@@ -534,7 +541,7 @@ def build_packed_plan(pb: GettProblem, prec: int, tile: int, groupM: int = 8,
     ident_m = np.arange(BM, dtype=np.int32)
     ident_n = np.arange(BN, dtype=np.int32)
     plan = GettPlan(pb, prec, tile, BM, BN, BK, lin_m, lin_n, lin_k, offAm, offAk, offBn, offBk, offCm, offCn,
-                    ident_m, ident_n, modeA, modeB, groupM, packed=True)
+                    ident_m, ident_n, modeA, modeB, groupM, packed=True, guard=guard)
     if store_waves:
         # store-wave kernel: persistent, one or two workgroups per CU by LDS
         if not sw_built(prec, tile):
@@ -789,26 +796,28 @@ def store_efficiency(segment_bytes: float) -> float:
 
 
 # Constants of the launch estimate, fitted (least squares on the logarithm,
-# plans near their contraction's best weighted up) to 17091 timed plans of 114
-# contractions: every pattern of tccg_amd.workloads over extents 8-72 (96-384
-# for the short-k pattern), every candidate plan.  The model's first choice
-# takes 1.03 (FP32), 1.02 (split-BF16), 1.04 (BF16), 1.03 (FP64) and 1.01 (FP8)
-# times the best candidate's time in the geometric mean, where the constants
-# before took 1.59, 1.42, 1.27, 1.15 and 1.06; the worst choice 1.39 times (5.2
-# before: store waves over a handful of tiles).
+# plans near their contraction's best weighted up) to timed plans: 17091 of 114
+# contractions, every pattern of tccg_amd.workloads over extents 8-72 (96-384
+# for the short-k pattern), every candidate plan; split-BF16 with its two sums
+# to 1300 plans of 104 contractions, 14 of them plain products that the fit did
+# not see.  The model's first choice takes 1.03 (FP32, FP64, split-BF16), 1.04
+# (BF16) and 1.01 (FP8) times the best candidate's time in the geometric mean,
+# at worst 1.53 times, and for the unseen products 1.01 (split-BF16).
 #
 # Packed kernels, per precision: MFMA time of a k-step over the nominal peak
 # (`mfma`), the share of the k-step's LDS traffic (128 bytes per clock) that the
 # MFMAs do not hide (`lds`), the shortest k-step of a workgroup in us (`step`),
 # a tile's prologue and epilogue in us (`tile`), the time of storing a tile over
 # what its CU's share of HBM bandwidth gives (`store`), and how much slower the
-# MFMAs run with every CU busy, where the power limit lowers the clock (`power`).
+# MFMAs run with every CU busy, where the power limit lowers the clock (`power`),
+# a persistent workgroup's time between tiles (`turn`) and how much longer a
+# tile's stores take where it is alone on its CU (`alone`).
 _PACKED_COST = {
-    F32: dict(mfma=1.08, lds=0.15, step=0.42, tile=2.0, store=0.18, power=0.04),
-    F64: dict(mfma=1.13, lds=0.3, step=0.23, tile=1.3, store=0.18, power=0.05),
-    BF16X3: dict(mfma=1.0, lds=0.29, step=0.36, tile=2.2, store=0.235, power=0.37),
-    FP8: dict(mfma=1.58, lds=0.0, step=0.07, tile=8.5, store=0.32, power=0.03),
-    BF16: dict(mfma=1.0, lds=0.35, step=0.21, tile=1.2, store=0.23, power=0.76),
+    F32: dict(mfma=1.08, lds=0.15, step=0.42, tile=2.0, store=0.18, power=0.04, alone=2.2, turn=0.3),
+    F64: dict(mfma=1.13, lds=0.3, step=0.23, tile=1.3, store=0.18, power=0.05, alone=2.2, turn=0.3),
+    BF16X3: dict(mfma=1.165, lds=0.137, step=0.317, tile=3.82, store=0.126, power=0.23, alone=4.0, turn=1.385),
+    FP8: dict(mfma=1.58, lds=0.0, step=0.07, tile=8.5, store=0.32, power=0.03, alone=2.2, turn=0.3),
+    BF16: dict(mfma=1.0, lds=0.35, step=0.21, tile=1.2, store=0.23, power=0.76, alone=2.2, turn=0.3),
 }
 # Gather kernels: the same, `scalar` the slowdown per operand read in a scalar
 # load mode, `walk` the us a persistent workgroup spends between tiles.
@@ -867,6 +876,8 @@ def _occupancy(plan: GettPlan) -> int:
         return 1 if area >= 128 * 128 else 2
     ring = packed_ring_bytes(plan.prec, plan.BM, plan.BN, plan.BK)
     by_regs = 1 if area >= 192 * 192 else 2 if area >= 128 * 128 else 4
+    if plan.prec == BF16X3:   # two accumulators per element
+        by_regs = 1 if area > 64 * 64 else 2
     return max(1, min(by_regs, MI355X["lds_bytes_per_cu"] // ring))
 
 
@@ -998,12 +1009,14 @@ def _estimate(plan: GettPlan, beta: float = 0.0) -> Tuple[float, float]:
             grid = max(1, min(plan.grid, cus * slots))
             j = max(1.0, grid / cus)
             # a run of C that the tile's m range cuts is written as partial lines
-            # by two workgroups (FP8's fitted store time holds it); a workgroup
+            # by two workgroups (FP8's fitted store time holds it; split-BF16's
+            # is fitted without it where a tile holds whole runs); a workgroup
             # alone on its CU has nothing to compute beside its stores
             run = _leading_run(plan.offCm[:4096].astype(np.int64), 1)
-            cut = 1.0 + 3.0 * run / plan.BM if run < plan.BM and plan.prec != FP8 else 1.0
-            out = (1.3 * j if j > 1 else 2.2) * cut * tile_store
-            gpu = -(-n // grid) * (steps * max(c["step"], j * step) + 0.3 + out) + c["tile"]
+            is_cut = run < plan.BM and plan.prec != FP8 and (plan.BM % run or plan.prec != BF16X3)
+            cut = 1.0 + 3.0 * run / plan.BM if is_cut else 1.0
+            out = (1.3 * j if j > 1 else c["alone"]) * cut * tile_store
+            gpu = -(-n // grid) * (steps * max(c["step"], j * step) + c["turn"] + out) + c["tile"]
         else:
             gpu = _rounds_us(n, slots, steps, step, c["step"], c["tile"], partial)
         if plan.ksplit > 1:
@@ -1042,45 +1055,50 @@ def candidate_plans(pb: GettProblem, prec: int, groupM: int = 8) -> List[GettPla
     return plans
 
 
-def _packed_candidates(pb: GettProblem, prec: int, groupM: int) -> List[GettPlan]:
-    """Every packed plan of candidate_plans()."""
+def _packed_candidates(pb: GettProblem, prec: int, groupM: int, guard: bool = False) -> List[GettPlan]:
+    """Every packed plan of candidate_plans() (guard: of split_plans())."""
     plans = []
-    for tile in range(len(PACKED_TILES[prec])):
-        plans.append(build_packed_plan(pb, prec, tile, groupM=groupM))
+    build = lambda tile, **kw: plans.append(build_packed_plan(pb, prec, tile, groupM=groupM, guard=guard, **kw))
+    for tile in SPLIT_RESIDENT if prec == BF16X3 else range(len(PACKED_TILES[prec])):
+        build(tile)
         if pb.K <= 256:
-            pp = build_packed_plan(pb, prec, tile, groupM=groupM, persistent=True)
-            if pp.grid:
-                plans.append(pp)
-        if sw_built(prec, tile):
-            plans.append(build_packed_plan(pb, prec, tile, groupM=groupM, store_waves=True))
+            build(tile, persistent=True)
+            if not plans[-1].grid:
+                plans.pop()
+        # (split-BF16: the persistent walk is as fast wherever store waves are,
+        # within 2 % over 104 contractions)
+        if prec != BF16X3 and sw_built(prec, tile):
+            build(tile, store_waves=True)
         # parallel-K when the tiles fill less than two rounds of the GPU and
         # k is long (the reference splits k when M*N is small next to the
         # threads, tccg/gett.py:933-936)
         BM, BN, BK = PACKED_TILES[prec][tile]
         kt = (-(-pb.K // BK) * BK) // BK
         nt = (-(-pb.M // BM)) * (-(-pb.N // BN))
-        if nt < 2 * MI355X["cus"] and kt >= 16:
+        if not guard and nt < 2 * MI355X["cus"] and kt >= 16:
             for ks in (2, 3, 4):
                 if ks <= kt // 8:
-                    plans.append(build_packed_plan(pb, prec, tile, groupM=groupM, ksplit=ks))
+                    build(tile, ksplit=ks)
         # stream-k when whole rounds of tiles would leave CUs idle in the last
         # one: few rounds, a partial last round, and k long enough that the
         # pieces stay long (under one round, k long enough to give every
         # workgroup a few k-steps of a tile)
-        if ((MI355X["cus"] <= nt < 8 * MI355X["cus"] and nt % MI355X["cus"] and kt >= 8)
-                or (nt < MI355X["cus"] and nt * kt >= 8 * MI355X["cus"])):
-            plans.append(build_packed_plan(pb, prec, tile, groupM=groupM, stream_k=1))
-            if packed_ring_bytes(prec, BM, BN, BK) * 2 <= MI355X["lds_bytes_per_cu"]:
-                plans.append(build_packed_plan(pb, prec, tile, groupM=groupM, stream_k=2))
+        # (split-BF16 over 192x64 never the fastest: 5184 x 1024, k = 5184: 405 us,
+        # 308 over 192x128)
+        if ((prec != BF16X3 or BM == BN or BM * BN > 192 * 64)
+                and ((MI355X["cus"] <= nt < 8 * MI355X["cus"] and nt % MI355X["cus"] and kt >= 8)
+                     or (nt < MI355X["cus"] and nt * kt >= 8 * MI355X["cus"]))):
+            build(tile, stream_k=1)
+            if prec != BF16X3 and packed_ring_bytes(prec, BM, BN, BK) * 2 <= MI355X["lds_bytes_per_cu"]:
+                build(tile, stream_k=2)
     return plans
 
 
 # Shortest k range of the plans that compute FP32 contractions on the BF16
-# MFMAs.  Their 2-norm error against FP64 is 0.45-0.88 times the FP32 MFMA's
-# for uniform, N(0, 1), positive and integer operands at every k from 4 to 5184
-# (measured; 1.25-1.4 times at k = 1, where the BF16 MFMA's truncated last
-# addition shows), and below 32 k values the packing costs more than the
-# faster instruction gains.
+# MFMAs: below 32 k values the packing costs more than the faster instruction
+# gains.  Their 2-norm error against FP64 is 0.09-0.69 times the FP32 MFMA's for
+# dense operands, uniform, N(0, 1) or positive, and with s nonzero values in a
+# row of A 1.02-1.03 times at s = 1, 0.83-0.91 at 2 and less from there on.
 SPLIT_MIN_K = 32
 
 
@@ -1117,12 +1135,9 @@ def split_plans(pb: GettProblem, groupM: int = 8) -> List[GettPlan]:
     is not held (include/tccg_gfx950.h, tccg_gett_f32_split)."""
     if pb.K < SPLIT_MIN_K:
         return []
-    plans = [p for p in _packed_candidates(pb, BF16X3, groupM)
-             if p.walk in (0, 5) and p.ksplit == 1 and split_fits(p)]
+    plans = [p for p in _packed_candidates(pb, BF16X3, groupM, guard=True) if split_fits(p)]
     bound = _chain_bound(pb)
     plans = [p for p in plans if _chain(p) <= bound]
-    for p in plans:
-        p.guard = True
     plans.sort(key=lambda p: _estimate(p))
     return plans
 
@@ -1132,9 +1147,16 @@ def call_plan(pb: GettProblem, prec: int) -> GettPlan:
     FP32 also the plans that compute it on the BF16 MFMAs."""
     best = default_plan(pb, prec)
     split = split_plans(pb)[:1] if prec == F32 else []
-    if split and _chain(best) > _chain_bound(pb):
+    if split and (_chain(best) > _chain_bound(pb) or _estimate(split[0]) <= _prefer_split(_estimate(best))):
         return split[0]
-    return min([best] + split, key=lambda p: _estimate(p))
+    return best
+
+
+def _prefer_split(estimate: Tuple[float, float]) -> Tuple[float, float]:
+    """FP32 plans have to be estimated 25 % faster to be chosen over a split plan:
+    over 104 contractions (90 of the workloads' patterns, 14 plain products) the
+    choice is then 1.012 times the best plan's time, 1.015 without."""
+    return tuple(1.25 * t for t in estimate)
 
 
 def default_plan(pb: GettProblem, prec: int) -> GettPlan:

@@ -8,7 +8,7 @@ import pytest
 
 from oracle.precision_ref import split_bf16_parts
 from tccg_amd import Contraction, build
-from tccg_amd.plan import (BF16X3, F32, F64, PACKED_TAIL_BYTES, SPLIT_MIN_K, build_packed_plan, call_plan,
+from tccg_amd.plan import (BF16X3, F32, F64, PACKED_TAIL_BYTES, PACKED_TILES, SPLIT_MIN_K, build_packed_plan, call_plan,
                            default_plan, split_plans)
 
 
@@ -73,8 +73,7 @@ def test_workspace_holds_the_guard_words(m, n, k):
     pb = _matmul(m, n, k).problem
     for t, kw in ((0, {}), (4, {}), (5, dict(stream_k=1)), (6, dict(persistent=True))):
         plain = build_packed_plan(pb, BF16X3, t, **kw)
-        p = build_packed_plan(pb, BF16X3, t, **kw)
-        p.guard = True
+        p = build_packed_plan(pb, BF16X3, t, guard=True, **kw)
         cp = _CPlan()
         cp.Mp, cp.Np, cp.Kp, cp.tile, cp.walk, cp.grid = p.Mp, p.Np, p.Kp, p.tile, p.walk, p.grid
         assert lib.tccg_f32_split_workspace_bytes(ctypes.byref(cp)) == p.workspace_bytes()
@@ -83,6 +82,12 @@ def test_workspace_holds_the_guard_words(m, n, k):
         # after every byte of the split-BF16 plan's, before the prefetch's tail
         assert off % 256 == 0 and off >= plain.workspace_bytes() - PACKED_TAIL_BYTES
         assert off + 256 + 4 * words <= p.workspace_bytes() - PACKED_TAIL_BYTES
+    for t in (7, 8):
+        p = build_packed_plan(pb, BF16X3, t, guard=True)
+        assert (p.BM, p.BN, p.BK) == PACKED_TILES[BF16X3][t] and p.Mp % p.BM == p.Np % p.BN == 0
+        cp = _CPlan()
+        cp.Mp, cp.Np, cp.Kp, cp.tile, cp.walk, cp.grid = p.Mp, p.Np, p.Kp, p.tile, p.walk, p.grid
+        assert lib.tccg_f32_split_workspace_bytes(ctypes.byref(cp)) == p.workspace_bytes()
 
 
 def test_operands_beyond_the_packed_limit_keep_the_fp32_plan():

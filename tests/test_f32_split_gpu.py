@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 
 from tccg_amd import Contraction
-from tccg_amd.plan import BF16X3, F32, PACKED_TILES, build_packed_plan
+from tccg_amd.plan import BF16X3, F32, PACKED_TILES, SPLIT_RESIDENT, build_packed_plan
 
 from .gpu_helpers import inputs, run_gpu
 
@@ -19,9 +19,7 @@ def _matmul(m, n, k):
 
 
 def _split(c, tile, **kw):
-    p = build_packed_plan(c.problem, BF16X3, tile, **kw)
-    p.guard = True
-    return p
+    return build_packed_plan(c.problem, BF16X3, tile, guard=True, **kw)
 
 
 def _exact(A, B, C, alpha, beta):
@@ -134,7 +132,7 @@ def test_zeros_have_the_sign_of_the_fp32_kernel(alpha, raw):
     fp32 = run_gpu(c, A, B, C, prec=F32, alpha=alpha, plan=build_packed_plan(c.problem, F32, 2))
     assert np.count_nonzero(fp32 == 0) > fp32.size // 8
     runs = 0
-    for tile, kw in [(0, {}), (6, {}), (0, WALKS[1]), (6, WALKS[1]), (4, WALKS[2])]:
+    for tile, kw in [(0, {}), (6, {}), (8, {}), (0, WALKS[1]), (6, WALKS[1]), (4, WALKS[2]), (7, WALKS[2])]:
         plan = _split(c, tile, **kw)
         runs += plan.crun[0] > 0 and not plan.grid
         out = run_gpu(c, A, B, C, prec=F32, alpha=alpha, plan=plan)
@@ -166,7 +164,7 @@ def test_raw_steps_over_long_k(walk, where):
         A *= np.float32(2.0 ** 45)
         if where == "both":
             B *= np.float32(2.0 ** 45)
-    for tile in (0, 4, 6):
+    for tile in SPLIT_RESIDENT:
         plan = _split(c, tile, **WALKS[walk])
         print(plan.describe(), flush=True)
         out = run_gpu(c, A, B, np.zeros(c.shapes()[2], np.float32), prec=F32, plan=plan)
@@ -191,16 +189,41 @@ def test_products_at_the_bottom_of_the_range(ea, eb):
     assert split <= fp32 + 2.0 ** -150
 
 
+def _errors(k, dist, nonzero=None, tiles=SPLIT_RESIDENT):
+    """2-norm errors of the split, tile by tile, and of the FP32 kernel; nonzero:
+    that many values in a row of A, at random places."""
+    c = _matmul(384, 320, k)
+    A, B, C = inputs(c, k + 7 * (nonzero or 0), dist)
+    if nonzero:
+        rng = np.random.default_rng(k)
+        A[np.argsort(rng.random(A.shape), axis=1) >= nonzero] = 0
+    ref, _ = _exact(A, B, C, 1.0, 0.0)
+    err = lambda plan: np.linalg.norm(run_gpu(c, A, B, C, prec=F32, plan=plan) - ref) / np.linalg.norm(ref)
+    split, fp32 = [err(_split(c, t)) for t in tiles], err(build_packed_plan(c.problem, F32, 2))
+    print("k %d %s %s: split %s, FP32 MFMA %.3e" % (k, dist, nonzero, ["%.3e" % e for e in split], fp32), flush=True)
+    return split, fp32
+
+
 @pytest.mark.parametrize("k", [32, 100, 2304])
 @pytest.mark.parametrize("dist", ["uniform", "normal"])
 def test_error_no_larger_than_the_fp32_kernels(k, dist):
-    c = _matmul(384, 320, k)
-    A, B, C = inputs(c, k, dist)
-    ref, _ = _exact(A, B, C, 1.0, 0.0)
-    err = lambda plan: np.linalg.norm(run_gpu(c, A, B, C, prec=F32, plan=plan) - ref) / np.linalg.norm(ref)
-    split, fp32 = err(_split(c, 0)), err(build_packed_plan(c.problem, F32, 2))
-    print("k %d %s: split %.3e, FP32 MFMA %.3e" % (k, dist, split, fp32), flush=True)
-    assert split <= fp32
+    """Dense operands: one rounding in the larger sum for 16 k values, where the
+    FP32 MFMA rounds once for two: from k = 32 on well under its error."""
+    split, fp32 = _errors(k, dist)
+    assert all(e <= 0.6 * fp32 for e in split)
+
+
+@pytest.mark.parametrize("k", [32, 512])
+@pytest.mark.parametrize("nonzero", [1, 2, 4, 8, 32])
+@pytest.mark.parametrize("dist", ["uniform", "normal"])
+def test_error_of_sums_of_few_products(k, nonzero, dist):
+    """Rows of A with few nonzero values.  One product is rounded once either way;
+    the split leaves out three part products of at most 2^-25 of it each, 0.41
+    units of the rounding's 0.58 at most, so sqrt(1 + 0.41^2 / 3) = 1.03 times the
+    error at one value (the left out products are uniform in their range), and no
+    more than the FP32 MFMA's from two values on."""
+    split, fp32 = _errors(k, dist, nonzero, (0, 7))
+    assert all(e <= (1.05 if nonzero == 1 else 1.0) * fp32 for e in split)
 
 
 def test_prepacked_call_and_reuse_of_a_workspace():
