@@ -1118,13 +1118,59 @@ def _chain(plan: GettPlan) -> float:
 
 
 def _chain_bound(pb: GettProblem) -> float:
-    """Longest summation chain of plans that calls in FP32 take: 1.3 times that
-    of FP32 stream-k over 128x128 tiles, which spreads k over the GPU where the
-    tiles are few.  The error grows with the chain's square root and the split's
-    is 0.87 times FP32's at equal chains, so no call is less exact than there
-    (one-tile split plans of 2401 x 221, k 3124: 7.6e-7 against 3.8e-7)."""
+    """Longest summation chain of split plans: 1.3 times that of FP32 stream-k
+    over 128x128 tiles, which spreads k over the GPU where the tiles are few, 512
+    at least."""
     tiles = -(-pb.M // 128) * (-(-pb.N // 128))
     return max(512.0, 1.3 * pb.K * min(1.0, tiles / MI355X["cus"]))
+
+
+# k values per rounding at full size of a sum: one MFMA of 2 (FP32) or 4 (FP64)
+# values; in split-BF16's larger sum one of 16.
+_PER_ROUNDING = {F32: 2.0, F64: 4.0, BF16X3: 16.0}
+
+
+def _roundings(plan: GettPlan) -> float:
+    """Roundings at full size on the way to an element of C: those of the longest
+    chain that a workgroup adds up, one per chain after that, and one for
+    split-BF16's two sums.  The error against exact sums of random operands is
+    2.5e-8 times the root of this count for every FP32 and split-BF16 plan
+    measured (k 256 to 4096, chains of 36 to 4096), 6.5e-17 in FP64."""
+    if plan.walk == 3:
+        return plan.problem.K
+    chain = max(1.0, _chain(plan))
+    return (chain / _PER_ROUNDING[plan.prec] + math.ceil(plan.problem.K / chain - 1e-9)
+            + (1 if plan.prec == BF16X3 else 0))
+
+
+# Counts that are precise enough without cutting k.
+_FEW_ROUNDINGS = {F32: 150.0, F64: 28.0, BF16X3: 100.0}
+
+
+def _roundings_bound(pb: GettProblem, prec: int) -> float:
+    """Most roundings of a plan that is chosen without a measurement, so that no
+    contraction's chains get longer because the estimate finds longer ones faster:
+    those of stream-k over 128x128 tiles (192x192 where these pad less and cut k
+    finer; 64x64 where the tiles are too few or k too short for either), which
+    spreads k over the GPU where the tiles are few.  Split-BF16 counts six
+    roundings per 16 k values in this bound, as in one sum."""
+    per = 16.0 / 6.0 if prec == BF16X3 else _PER_ROUNDING[prec]
+    tiles = lambda t: -(-pb.M // t) * (-(-pb.N // t))
+
+    def stream_k(t, bk, grid):
+        n, kt, cus = tiles(t), -(-pb.K // bk), MI355X["cus"]
+        if not (n * kt >= 8 * cus if n < cus else n < 8 * cus and n % cus and kt >= 8):
+            return math.inf
+        chain = pb.K * min(1.0, n / grid)
+        return chain / per + math.ceil(pb.K / chain - 1e-9)
+
+    cus = MI355X["cus"]
+    bound = stream_k(128, 16, cus)
+    if prec != F64 and tiles(192) * 192 ** 2 < tiles(128) * 128 ** 2:
+        bound = min(bound, stream_k(192, 16, cus))
+    if bound == math.inf and prec != F32:
+        bound = stream_k(64, 16 if prec == F64 else 32, 2 * cus)
+    return max(bound, _FEW_ROUNDINGS[prec])
 
 
 def split_plans(pb: GettProblem, groupM: int = 8) -> List[GettPlan]:
@@ -1160,4 +1206,10 @@ def _prefer_split(estimate: Tuple[float, float]) -> Tuple[float, float]:
 
 
 def default_plan(pb: GettProblem, prec: int) -> GettPlan:
-    return candidate_plans(pb, prec)[0]
+    """The model's best candidate plan (FP32, FP64 and split-BF16: of those within
+    _roundings_bound(), or the one with the fewest roundings)."""
+    plans = candidate_plans(pb, prec)
+    if prec not in _PER_ROUNDING:
+        return plans[0]
+    bound = _roundings_bound(pb, prec)
+    return next((p for p in plans if _roundings(p) <= bound), min(plans, key=_roundings))

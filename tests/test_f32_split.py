@@ -134,3 +134,58 @@ def test_calls_do_not_lengthen_the_summation_chains(m, n, k):
         assert call_plan(pb, F32).describe() == default_plan(pb, F32).describe()
     for p in split and [call_plan(pb, F32)] + split:
         assert _chain(p) <= max(512, 1.3 * k * min(1.0, tiles / 256)), p.describe()
+
+
+# (m, n, k) of a product and the full-size roundings of the plans that were chosen
+# for it in FP32, FP64 and split-BF16 when the launch estimate was fitted to larger
+# tiles and stream-k (split-BF16: six per 16 k values, in one sum).
+ROUNDINGS = [
+    (930, 840, 4002, 446, 226, 336),
+    (1152, 640, 896, 449, 46, 337),
+    (2414, 598, 1420, 271, 137, 204),
+    (1840, 1460, 480, 241, 87, 181),
+    (930, 3264, 2296, 387, 470, 704),
+    (2296, 930, 3264, 388, 461, 691),
+    (221, 3124, 2401, 244, 125, 185),
+    (247, 840, 4200, 2101, 77, 1576),
+    (4200, 247, 840, 421, 60, 316),
+    (480, 1496, 1554, 778, 80, 584),
+    (2150, 494, 2688, 361, 183, 272),
+    (2520, 352, 1536, 769, 95, 140),
+    (3192, 275, 2691, 403, 204, 303),
+    (1976, 558, 986, 494, 82, 205),
+    (3332, 1725, 1200, 387, 301, 451),
+    (4980, 1344, 2679, 958, 671, 719),
+    (3149, 2076, 3344, 1230, 837, 923),
+    (1320, 800, 190, 96, 28, 73),
+    (726, 840, 431, 217, 40, 163),
+    (312, 1848, 672, 337, 52, 253),
+    (64, 64, 20000, 10001, 1254, 7501),
+    (128, 128, 32, 17, 9, 13),
+    (300, 300, 511, 257, 36, 193),
+    (5184, 5184, 2304, 1153, 577, 865),
+    (99, 810, 1450, 726, 48, 545),
+    (2065, 493, 3654, 493, 249, 371),
+    (583, 1788, 3273, 455, 230, 342),
+    (48, 48, 48, 25, 13, 19),
+]
+
+
+@pytest.mark.parametrize("m, n, k, f32, f64, bf16x3", ROUNDINGS)
+def test_no_plan_rounds_more_often_than_those_chosen_before(m, n, k, f32, f64, bf16x3):
+    """The plans of calls and of the code generators: the error grows with the root
+    of the count, 3 % of it is the allowance for padded k-steps."""
+    from tccg_amd.plan import _roundings
+    pb = _matmul(m, n, k).problem
+    for prec, before in ((F32, f32), (F64, f64), (BF16X3, bf16x3)):
+        for plan in (default_plan(pb, prec), call_plan(pb, prec)):
+            assert _roundings(plan) <= 1.03 ** 2 * before, plan.describe()
+
+
+def test_roundings_of_a_plan():
+    from tccg_amd.plan import _roundings
+    pb = _matmul(256, 256, 1024).problem
+    assert _roundings(build_packed_plan(pb, F32, 0)) == 1024 / 2 + 1
+    assert _roundings(build_packed_plan(pb, F32, 0, ksplit=4)) == 256 / 2 + 4
+    assert _roundings(build_packed_plan(pb, F64, 0, stream_k=1)) == 1024 * 4 / 256 / 4 + 64   # 4 tiles on 256
+    assert _roundings(build_packed_plan(pb, BF16X3, 0)) == 1024 / 16 + 1 + 1
