@@ -67,6 +67,9 @@ enum tccg_load_mode { TCCG_FREE4 = 0, TCCG_FREE1 = 1, TCCG_KDIM4 = 2, TCCG_KDIM1
  * ordA/ordB (device int32, lengths BM/BN) give the tile row filled by each
  * loader slot, so that the lanes of a wave can walk an operand's stride-one
  * index; use the identity when no reordering is wanted.
+ * A, B and C may start at any element: a pointer off the 16-byte boundary is
+ * read or written one element at a time where the plan would use 16-byte
+ * accesses (the same sums, slower), gather plans then on the one-tile walk.
  */
 typedef struct tccg_gett_plan {
   const uint32_t* offAm;
@@ -120,9 +123,9 @@ typedef struct tccg_gett_plan {
   int32_t crun_n;      /* C's stride-one index spans crun_m consecutive m   */
                        /* positions and C's next index crun_n consecutive n */
                        /* positions (offCm[m + a] = offCm[m] + a,           */
-                       /* offCn[n + b] = offCn[n] + b * crun_m), tiles hold */
-                       /* whole blocks and C is 16-byte aligned: the tile   */
-                       /* is written as crun_m * crun_n element runs.       */
+                       /* offCn[n + b] = offCn[n] + b * crun_m) and tiles   */
+                       /* hold whole blocks: the tile is written as         */
+                       /* crun_m * crun_n element runs.                     */
                        /* 0 for the plain epilogue.  Walk 4: crun_m > 0     */
                        /* selects the run store order: every aligned run of */
                        /* crun_m m positions (a multiple of 4 dividing BM)  */

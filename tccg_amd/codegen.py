@@ -95,9 +95,16 @@ def emit_source(plan: GettPlan, contraction_text: str, name: str = "gett") -> st
     WM, WN = WAVES.get((plan.prec, plan.tile), (2, 2))
     walk = 2 if plan.walk == 2 else (1 if plan.grid else 0)
     vector = plan.walk == 3
+    # Pointers off the 16-byte boundary: gather and vector plans have a second
+    # kernel that reads and writes one element at a time (the same tables, tiles
+    # and order of sums), packed plans drop the 16-byte stores of C.
+    scalar = None
     if vector:
         kern = "tccg::gett_vector_kernel<%s, %d, %d, %d, %d>" % (
             _PREC_ENUM[plan.prec], plan.BM, plan.BN, plan.BK, 4 if plan.modeA == 0 else 1)
+        if plan.modeA == 0:
+            scalar = "tccg::gett_vector_kernel<%s, %d, %d, %d, 1>" % (
+                _PREC_ENUM[plan.prec], plan.BM, plan.BN, plan.BK)
         shape = "void"   # no tile shape: the kernel's LDS is static
     elif plan.packed and plan.walk == 4:
         WM, WN = 2, 2
@@ -119,6 +126,9 @@ def emit_source(plan: GettPlan, contraction_text: str, name: str = "gett") -> st
     else:
         kern = "tccg::gett_kernel<%s, %d, %d, %d, %d, %d, %d, %d, %d>" % (
             _PREC_ENUM[plan.prec], plan.BM, plan.BN, plan.BK, WM, WN, plan.modeA, plan.modeB, walk)
+        if plan.modeA in (0, 2) or plan.modeB in (0, 2):
+            scalar = "tccg::gett_kernel<%s, %d, %d, %d, %d, %d, %d, %d, 0>" % (
+                _PREC_ENUM[plan.prec], plan.BM, plan.BN, plan.BK, WM, WN, plan.modeA | 1, plan.modeB | 1)
         shape = "tccg::TileShape<%s, %d, %d, %d, %d, %d>" % (_PREC_ENUM[plan.prec], plan.BM, plan.BN, plan.BK, WM, WN)
     desc = contraction_text.strip().replace("\\", "\\\\").replace('"', '\\"').replace("\n", "\\n")
     swap = "1" if pb.swapped else "0"
@@ -231,32 +241,46 @@ __global__ void amax_reduce(const float* __restrict__ x, int64_t n, unsigned* o)
         lds = "S::LDS_BYTES / 2"   # a single k-step never touches the second stage
     else:
         lds = "S::LDS_BYTES"
-    out.append(("""  using S = %s;
-  constexpr int kLds = """ + lds + """;
+    single = "S::LDS_BYTES / 2" if plan.Kp == plan.BK else "S::LDS_BYTES"   # one k-step: one stage
+    checks, when = [], []
+    if not plan.packed and plan.modeA in (0, 2):
+        checks.append("opA")
+        when.append("operand A of the GETT must be 16-byte aligned")
+    if not plan.packed and not vector and plan.modeB in (0, 2):
+        checks.append("opB")
+        when.append("operand B of the GETT must be 16-byte aligned")
+    if (vector and plan.modeA == 0) or (plan.packed and (plan.cvec or plan.crun[0])):
+        checks.append("C")
+        when.append("C must be 16-byte aligned")
+    off = " | ".join("reinterpret_cast<uintptr_t>(%s)" % x for x in checks)
+    out.append("""  using S = %s;
   if (!A || !B || !C) return fail(1, "tensor pointer is NULL");
   DeviceTables* t = nullptr;
   int rc = tables_for_current_device(&t);
   if (rc) return rc;
+  const %s* opA = %s ? B : A;
+  const %s* opB = %s ? A : B;
   auto kern = %s;
-  // the dynamic-LDS limit is a per-device attribute: one bit per device id
-  static std::atomic<uint64_t> lds_set{0};
+  int kLds = %s, grid = %d;
+""" % (shape, T, swap, T, swap, kern, lds, plan.grid if plan.grid else plan.ntiles() * plan.ksplit))
+    if checks:
+        out.append("  // for 16-byte accesses %s; else one element at a time\n"
+                   "  const bool off16 = ((%s) & 15u) != 0;\n" % (", ".join(when), off))
+    if scalar:
+        out.append("  if (off16) { kern = %s; kLds = %s; grid = %d; }\n"
+                   % (scalar, "0" if vector else single, plan.ntiles()))
+    out.append("""  // the dynamic-LDS limit is a per-device attribute: one bit per device id
+  static std::atomic<uint64_t> lds_set[2];
+  std::atomic<uint64_t>& lds_done = lds_set[%s];
   int lds_dev = 0;
   if (hipGetDevice(&lds_dev) != hipSuccess) return fail(1, "hipGetDevice failed");
   const uint64_t dev_bit = lds_dev < 64 ? (uint64_t{1} << lds_dev) : 0;
-  if (!dev_bit || !(lds_set.load(std::memory_order_acquire) & dev_bit)) {
+  if (!dev_bit || !(lds_done.load(std::memory_order_acquire) & dev_bit)) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
     if (e != hipSuccess) return fail((int)e, std::string("hipFuncSetAttribute: ") + hipGetErrorString(e));
-    lds_set.fetch_or(dev_bit, std::memory_order_release);
+    lds_done.fetch_or(dev_bit, std::memory_order_release);
   }
-  const %s* opA = %s ? B : A;
-  const %s* opB = %s ? A : B;
-""") % (shape, kern, T, swap, T, swap))
-    if not plan.packed and plan.modeA in (0, 2):
-        out.append('  if (reinterpret_cast<uintptr_t>(opA) & 15u) return fail(1, "operand A of the GETT must be 16-byte aligned");\n')
-    if not plan.packed and plan.modeB in (0, 2):
-        out.append('  if (reinterpret_cast<uintptr_t>(opB) & 15u) return fail(1, "operand B of the GETT must be 16-byte aligned");\n')
-    if (vector and plan.modeA == 0) or (plan.packed and (plan.cvec or plan.crun[0])):
-        out.append('  if (reinterpret_cast<uintptr_t>(C) & 15u) return fail(1, "C must be 16-byte aligned");\n')
+""" % ("off16 ? 1 : 0" if scalar else "0"))
     out.append("  hipStream_t s = (hipStream_t)stream;\n")
     if plan.prec == FP8:
         out.append("""  hipLaunchKernelGGL(amax_zero, dim3(1), dim3(64), 0, s, reinterpret_cast<unsigned*>(t->amax));
@@ -295,20 +319,21 @@ __global__ void amax_reduce(const float* __restrict__ x, int64_t n, unsigned* o)
   p.tilesM = %d; p.tilesN = %d; p.kTiles = %d; p.groupM = %d;
   p.alpha = alpha; p.beta = beta;
   p.amax = %s;
-  p.crunM = %d; p.crunN = %d; p.cvec = %d;
+  p.crunM = %s; p.crunN = %s; p.cvec = %s;
   p.ksplit = %d; p.part = %s; p.flags = %s;
-  hipLaunchKernelGGL(kern, dim3(%d), dim3(%d), kLds, s, p);
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(%d), kLds, s, p);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail((int)e, std::string("kernel launch: ") + hipGetErrorString(e));
 %s  return 0;
 }
 
 """ % (T, plan.Mp // plan.BM, plan.Np // plan.BN, plan.Kp // plan.BK, plan.groupM,
-       "t->amax" if plan.prec == FP8 else "nullptr", plan.crun[0], plan.crun[1], plan.cvec,
+       "t->amax" if plan.prec == FP8 else "nullptr",
+       *(("off16 ? 0 : %d" % v if plan.packed and v else "%d" % v) for v in (*plan.crun, plan.cvec)),
        plan.ksplit, _part_expr(plan, T),
        ("reinterpret_cast<uint32_t*>(reinterpret_cast<unsigned char*>(t->ws) + %d)" % _flags_offset(plan)
         if plan.walk == 5 else "nullptr"),
-       plan.grid if plan.grid else plan.ntiles() * plan.ksplit, 512 if plan.walk == 4 else 256,
+       512 if plan.walk == 4 else 256,
        _reduce_launch(plan, T)))
     out.append("void gett({T}* A, {T}* B, {T}* C, const {T} alpha, const {T} beta) {{\n"
                "  (void)gett_stream(A, B, C, alpha, beta, nullptr);\n}}\n\n".format(T=T))

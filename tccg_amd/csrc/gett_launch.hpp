@@ -235,6 +235,12 @@ int dispatch_tile(int tile, int ma, int mb, const tccg::GettParams<typename tccg
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
+// The load mode for operand X: vector modes need a 16-byte aligned pointer.
+inline int scalar_mode(int mode, const void* X) {
+  if (aligned16(X)) return mode;
+  return mode == TCCG_FREE4 ? TCCG_FREE1 : mode == TCCG_KDIM4 ? TCCG_KDIM1 : mode;
+}
+
 // Vector micro-kernel tile I (or a later one) of precision P.
 template <int P, int I>
 int dispatch_vector_tile(int tile, int vec, const tccg::GettParams<typename tccg::PrecTraits<P>::TG>& prm,
@@ -273,10 +279,10 @@ int run_gett(const typename tccg::PrecTraits<P>::TG* A, const typename tccg::Pre
   if (!plan->offAm || !plan->offAk || !plan->offBn || !plan->offBk || !plan->offCm || !plan->offCn ||
       !plan->ordA || !plan->ordB)
     return fail(1, "offset or order table pointer is NULL");
-  const bool vecA = plan->modeA == TCCG_FREE4 || plan->modeA == TCCG_KDIM4;
-  const bool vecB = plan->modeB == TCCG_FREE4 || plan->modeB == TCCG_KDIM4;
-  if ((vecA && !aligned16(A)) || (vecB && !aligned16(B)))
-    return fail(1, "vector load mode requires 16-byte aligned operands");
+  // An operand off the 16-byte boundary is read one element at a time: the same
+  // tables, tiles and order of sums, so the same bits, on the one-tile walk.
+  const int modeA = scalar_mode(plan->modeA, A), modeB = scalar_mode(plan->modeB, B);
+  const bool moved = modeA != plan->modeA || modeB != plan->modeB;
   const TileCfg& tc = tiles[plan->tile];
   if (plan->Mp % tc.BM || plan->Np % tc.BN || plan->Kp % tc.BK)
     return fail(1, "table lengths must be whole multiples of the tile shape");
@@ -306,9 +312,7 @@ int run_gett(const typename tccg::PrecTraits<P>::TG* A, const typename tccg::Pre
     // modeA FREE4: groups of four m positions contiguous in A and in C
     if (plan->Kp != tc.BK) return fail(1, "the vector micro-kernel needs the whole k range in one tile (Kp == BK)");
     if (plan->grid != 0) return fail(1, "the vector micro-kernel runs one workgroup per tile (grid 0)");
-    const int vec = plan->modeA == TCCG_FREE4 ? 4 : 1;
-    if (vec == 4 && (!aligned16(A) || !aligned16(C)))
-      return fail(1, "the vector micro-kernel with four-wide groups needs 16-byte aligned A and C");
+    const int vec = modeA == TCCG_FREE4 && aligned16(C) ? 4 : 1;
     if constexpr (P == tccg::F32 || P == tccg::F64) {
       return dispatch_vector_tile<P, 0>(plan->tile, vec, prm, (hipStream_t)stream);
     }
@@ -322,7 +326,8 @@ int run_gett(const typename tccg::PrecTraits<P>::TG* A, const typename tccg::Pre
                      4L * ((long)prm.tilesN * tc.BN + tc.BM);
     if (lds > kMaxLds) return fail(1, "the streaming walk needs B's n-tiles and A's tile in LDS (too large)");
   }
-  return dispatch_tile<P>(plan->tile, plan->modeA, plan->modeB, prm, plan->grid, plan->walk, (hipStream_t)stream);
+  return dispatch_tile<P>(plan->tile, modeA, modeB, prm, moved ? 0 : plan->grid, moved ? 0 : plan->walk,
+                          (hipStream_t)stream);
 }
 
 
@@ -659,9 +664,10 @@ int run_gett_packed(const typename tccg::PrecTraits<P>::TG* A, const typename tc
   prm.groupM = plan->groupM > 0 ? plan->groupM : 1;
   prm.alpha = alpha; prm.beta = beta;
   prm.amax = plan->amax;
-  prm.crunM = plan->crun_m;
-  prm.crunN = plan->crun_n;
-  prm.cvec = plan->cvec;
+  // (C off the 16-byte boundary is written one element at a time)
+  prm.crunM = aligned16(C) ? plan->crun_m : 0;
+  prm.crunN = aligned16(C) ? plan->crun_n : 0;
+  prm.cvec = aligned16(C) ? plan->cvec : 0;
   prm.ksplit = plan->ksplit > 1 ? plan->ksplit : 1;
   prm.part = reinterpret_cast<TG*>(reinterpret_cast<unsigned char*>(workspace) + offP);
   prm.flags = plan->walk == 5 ? reinterpret_cast<uint32_t*>(reinterpret_cast<unsigned char*>(workspace) + offF)
@@ -693,7 +699,6 @@ int run_gett_packed(const typename tccg::PrecTraits<P>::TG* A, const typename tc
     if (plan->crun_m < 0 || plan->crun_m % 4 || (plan->crun_m > 0 && tc.BM % plan->crun_m))
       return fail(1, "walk 4: crun_m (the run length of the run store order) must be 0 or a multiple of 4 "
                      "that divides the tile's BM");
-    if ((plan->cvec || plan->crun_m) && !aligned16(C)) return fail(1, "16-byte stores need a 16-byte aligned C");
     if (!std::is_same<TG, float>::value) return fail(1, "the store-wave kernel (walk 4) writes FP32 results only");
   } else {
     if (plan->walk != 0 && plan->walk != 5) return fail(1, "packed plans take walk 0, 4 or 5");
@@ -704,8 +709,6 @@ int run_gett_packed(const typename tccg::PrecTraits<P>::TG* A, const typename tc
     }
     if (plan->crun_m < 0 || plan->crun_n < 0 || (plan->crun_m > 0) != (plan->crun_n > 0))
       return fail(1, "crun_m and crun_n must both be positive or both zero");
-    if (plan->crun_m > 0 && !aligned16(C))
-      return fail(1, "the run epilogue (crun_m > 0) needs a 16-byte aligned C");
   }
   if (pack) {
     // the stream-k flags start clear: the pack launch clears them
