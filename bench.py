@@ -291,7 +291,6 @@ def run_batch(args, log):
     import numpy as np
     import torch
     from tccg_amd.batch import GettBatch, autotune_group, random_batch
-    from tccg_amd.plan import F32, PACKED_TILES
     cs = random_batch(512, seed=0)
     rng = np.random.default_rng(0)
     As, Bs, Cs = [], [], []
@@ -325,7 +324,7 @@ def run_batch(args, log):
     flops = b.flops()
     grp = b._bound["group"]._bound
     res = {"workload": "512 FP32 contractions, 4 patterns, extents U{8..96 step 8}, seed 0",
-           "problems": len(cs), "launches_per_step": b.launches(), "tile": list(PACKED_TILES[F32][tile]),
+           "problems": len(cs), "launches_per_step": b.launches(), "tile": list(b.tile_shape()),
            "work_order": order, "work_items": grp["nwork"], "pack_jobs": grp["njobs"],
            "tune_seconds": round(tune_s, 2),
            "wall_ms_per_step": wall * 1e3, "kernel_ms": kern * 1e3, "gflops": flops / wall / 1e9,

@@ -114,6 +114,10 @@ class GettBatch:
     def _default_shape(c: Contraction) -> int:
         return 1 if c.problem.M * c.problem.N >= 256 * 256 else 0
 
+    def tile_shape(self):
+        """(BM, BN, BK) of the grouped launch (split-BF16's where it runs there)."""
+        return PACKED_TILES[self.plans[0].prec][self.plans[0].tile]
+
     def flops(self) -> float:
         return sum(c.flops(b) for c, b in zip(self.contractions, self.betas))
 
@@ -299,10 +303,12 @@ def group_candidates(contractions: Sequence[Contraction], betas: Optional[Sequen
     work orders."""
     from .plan import group_estimate
     betas = list(betas) if betas is not None else [c.beta for c in contractions]
-    est = []
+    # one candidate per launch: group_split_tile() maps several FP32 tiles to one
+    launches = {}
     for t in range(len(PACKED_TILES[F32])):
-        est.append((group_estimate(group_plans(contractions, t), betas), t))
-    est.sort()
+        plans = group_plans(contractions, t)
+        launches.setdefault(frozenset((p.prec, p.tile) for p in plans), (t, plans))
+    est = sorted((group_estimate(plans, betas), t) for t, plans in launches.values())
     # longest k range first balances the workgroups better than whole problems
     # per XCD: 4-9 % over batches of 8, 40 and 512 problems
     return [(t, order, e) for e, t in est for order in ("lpt", "xcd")]
@@ -330,7 +336,7 @@ def autotune_group(contractions: Sequence[Contraction], As, Bs, Cs, top: int = 6
         if verbose:
             import sys
             print("  group tile %s order %s: model %.2f ms, measured %.2f ms" % (
-                PACKED_TILES[F32][tile], order, est * 1e3, t * 1e3), file=sys.stderr)
+                b.tile_shape(), order, est * 1e3, t * 1e3), file=sys.stderr)
         if best is None or t < best[2]:
             best = (tile, order, t)
         del b

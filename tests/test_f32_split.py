@@ -189,3 +189,17 @@ def test_roundings_of_a_plan():
     assert _roundings(build_packed_plan(pb, F32, 0, ksplit=4)) == 256 / 2 + 4
     assert _roundings(build_packed_plan(pb, F64, 0, stream_k=1)) == 1024 * 4 / 256 / 4 + 64   # 4 tiles on 256
     assert _roundings(build_packed_plan(pb, BF16X3, 0)) == 1024 / 16 + 1 + 1
+
+
+@pytest.mark.parametrize("n, min_k", [(8, 8), (40, 8), (3, 1)])
+def test_group_candidates_are_different_launches(n, min_k):
+    """Each (tile, order) choice of a batch is a launch of its own, whether the
+    batch runs on the BF16 MFMAs or (a k range under four) on the FP32 ones."""
+    from tccg_amd.batch import group_candidates, group_plans, random_batch
+    cs = random_batch(n, seed=n)
+    if min_k < 4:
+        cs.append(_matmul(40, 30, min_k))
+    launches = [((group_plans(cs, t)[0].prec, group_plans(cs, t)[0].tile), order) for t, order, _ in group_candidates(cs)]
+    assert len(set(launches)) == len(launches) >= 8
+    every = {(p.prec, p.tile) for t in range(len(PACKED_TILES[F32])) for p in group_plans(cs, t)}
+    assert {l for l, _ in launches} == every   # and no launch is left out
