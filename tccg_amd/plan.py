@@ -1150,9 +1150,10 @@ _FEW_ROUNDINGS = {F32: 150.0, F64: 28.0, BF16X3: 100.0}
 def _roundings_bound(pb: GettProblem, prec: int) -> float:
     """Most roundings of a plan that is chosen without a measurement, so that no
     contraction's chains get longer because the estimate finds longer ones faster:
-    those of stream-k over 128x128 tiles (192x192 where these pad less and cut k
-    finer; 64x64 where the tiles are too few or k too short for either), which
-    spreads k over the GPU where the tiles are few.  Split-BF16 counts six
+    those of stream-k over 128x128 tiles (192x192 where these pad no more and cut k
+    finer; 64x64 where the tiles are too few or k too short for either, in FP64
+    two parts of k where they are for that), which spreads k over the GPU where the
+    tiles are few.  Split-BF16 counts six
     roundings per 16 k values in this bound, as in one sum."""
     per = 16.0 / 6.0 if prec == BF16X3 else _PER_ROUNDING[prec]
     tiles = lambda t: -(-pb.M // t) * (-(-pb.N // t))
@@ -1166,10 +1167,12 @@ def _roundings_bound(pb: GettProblem, prec: int) -> float:
 
     cus = MI355X["cus"]
     bound = stream_k(128, 16, cus)
-    if prec != F64 and tiles(192) * 192 ** 2 < tiles(128) * 128 ** 2:
+    if prec != F64 and tiles(192) * 192 ** 2 <= tiles(128) * 128 ** 2:
         bound = min(bound, stream_k(192, 16, cus))
     if bound == math.inf and prec != F32:
         bound = stream_k(64, 16 if prec == F64 else 32, 2 * cus)
+    if bound == math.inf and prec == F64 and pb.K > 240:
+        bound = -(-pb.K // 32) * 16 / per + 2   # two parts
     return max(bound, _FEW_ROUNDINGS[prec])
 
 
@@ -1212,4 +1215,5 @@ def default_plan(pb: GettProblem, prec: int) -> GettPlan:
     if prec not in _PER_ROUNDING:
         return plans[0]
     bound = _roundings_bound(pb, prec)
-    return next((p for p in plans if _roundings(p) <= bound), min(plans, key=_roundings))
+    # (6 %: pieces of whole k-steps, 3 % of error)
+    return next((p for p in plans if _roundings(p) <= 1.06 * bound), min(plans, key=_roundings))

@@ -168,6 +168,9 @@ ROUNDINGS = [
     (2065, 493, 3654, 493, 249, 371),
     (583, 1788, 3273, 455, 230, 342),
     (48, 48, 48, 25, 13, 19),
+    (480, 282, 269, 136, 38, 102),
+    (3392, 1815, 3087, 1093, 773, 1159),
+    (175, 1763, 358, 180, 50, 135),
 ]
 
 
