@@ -1196,16 +1196,20 @@ def call_plan(pb: GettProblem, prec: int) -> GettPlan:
     FP32 also the plans that compute it on the BF16 MFMAs."""
     best = default_plan(pb, prec)
     split = split_plans(pb)[:1] if prec == F32 else []
-    if split and (_chain(best) > _chain_bound(pb) or _estimate(split[0]) <= _prefer_split(_estimate(best))):
+    if split and (_chain(best) > _chain_bound(pb) or _estimate(split[0]) <= _prefer_split(best)):
         return split[0]
     return best
 
 
-def _prefer_split(estimate: Tuple[float, float]) -> Tuple[float, float]:
-    """FP32 plans have to be estimated 25 % faster to be chosen over a split plan:
-    over 104 contractions (90 of the workloads' patterns, 14 plain products) the
-    choice is then 1.012 times the best plan's time, 1.015 without."""
-    return tuple(1.25 * t for t in estimate)
+def _prefer_split(plan: GettPlan) -> Tuple[float, float]:
+    """What a split plan's estimate is compared with: that of the FP32 plan, which
+    has to be estimated 25 % faster to be chosen where it is packed too (the FP32
+    estimate of persistent plans is too low, C of 7038 x 8976, k = 56: 101 and 118
+    us estimated, 198 and 168 measured).  Not where it is a gather plan, one launch
+    less (2304 x 2304, k = 64: 13.6 and 15.7 us estimated, 15.0 and 15.8 measured):
+    over 20 contractions with one the choice is 1.007 times the best plan's time."""
+    f = 1.25 if plan.packed else 1.0
+    return tuple(f * t for t in _estimate(plan))
 
 
 def default_plan(pb: GettProblem, prec: int) -> GettPlan:
